@@ -494,7 +494,8 @@ def main():
     launches = stats[0]["launches"]
     dev_s = stats[0]["elapsed_ms"] / 1e3
     idx = max(workloads.index_bytes(q.n_nodes, args.slices_per_wave) for q in qps)
-    alg = sum(workloads.solve_bytes(q.qp.op_counts(), q.n_nodes, q.n_blocks, q.m, mixed, idx=idx) for q in qps)
+    alg = sum(workloads.solve_bytes(q.qp.op_counts(), q.n_nodes, q.n_blocks, q.m, mixed, idx=idx, moved=True)
+              for q in qps)
     achieved = alg / dev_s / 1e9
     roof = {"kernel": "mprgp_step", "bound": "hbm", "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),

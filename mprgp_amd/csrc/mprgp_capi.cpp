@@ -682,7 +682,7 @@ static int ensure_matrix32(mprgp_matrix *A, hipStream_t s) {
 static int ensure_qp32(mprgp_qp *q, hipStream_t s) {
   if (q->base32) return MPRGP_OK;
   const size_t n3 = 3 * (size_t)q->n;
-  const size_t bytes = (3 * n3 + (size_t)q->n) * sizeof(double) + (9 * n3 + 64) * sizeof(float);
+  const size_t bytes = (3 * n3 + (size_t)q->n) * sizeof(double) + (8 * n3 + 64) * sizeof(float);
   if (int rc = q->ctx->alloc(&q->base32, bytes)) return rc;
   q->bytes32 = bytes;
   double *dp = (double *)q->base32;
@@ -694,7 +694,7 @@ static int ensure_qp32(mprgp_qp *q, hipStream_t s) {
   q->fcc = dp;
   dp += q->n;
   float *fp32 = (float *)dp;
-  float **fvecs[] = {&q->fp, &q->fp2, &q->fz, &q->fap, &q->fb, &q->fg, &q->fphi, &q->fbeta, &q->fbeta2};
+  float **fvecs[] = {&q->fp, &q->fp2, &q->fz, &q->fap, &q->fb, &q->fg, &q->fbeta, &q->fbeta2};
   for (float **v : fvecs) {
     *v = fp32;
     fp32 += n3;
@@ -1484,7 +1484,7 @@ void describe_qp(const mprgp_qp *q, const mprgp_params &p, int n_tiles, int *don
   d.col16 = q->A->d_col16;
   d.d.val = q->A->d_val;
   d.d.dinv = q->A->d_dinv;
-  d.d.x = q->x; d.d.b = q->b; d.d.g = q->g; d.d.p = q->p; d.d.z = q->z; d.d.phi = q->phi;
+  d.d.x = q->x; d.d.b = q->b; d.d.g = q->g; d.d.p = q->p; d.d.z = q->z;
   d.d.beta = q->beta; d.d.y = q->y; d.d.ap = q->ap; d.d.py = q->py;
   d.d.p2 = q->p2; d.d.beta2 = q->beta2;
   d.d.cn = q->cn; d.d.cc = q->cc; d.d.cj = q->cj; d.d.cs = q->cs;
@@ -1494,7 +1494,7 @@ void describe_qp(const mprgp_qp *q, const mprgp_params &p, int n_tiles, int *don
   if (mixed) {
     d.f.val = q->A->d_val32;
     d.f.dinv = q->A->d_dinv;
-    d.f.x = q->fx; d.f.b = q->fb; d.f.g = q->fg; d.f.p = q->fp; d.f.z = q->fz; d.f.phi = q->fphi;
+    d.f.x = q->fx; d.f.b = q->fb; d.f.g = q->fg; d.f.p = q->fp; d.f.z = q->fz;
     d.f.beta = q->fbeta; d.f.y = q->fy; d.f.ap = q->fap; d.f.py = q->fpy; d.f.p2 = q->fp2;
     d.f.beta2 = q->fbeta2;
     d.f.cn = q->cn; d.f.cj = q->cj; d.f.cs = q->cs; d.f.cc = q->fcc;

@@ -117,7 +117,7 @@ static_assert(sizeof(QpState) == 8 * kSlice, "QpState must stay 512 bytes");
 
 // Storage of one precision form: FP64 for the plain solve and the outer
 // refinement; for the inner solve of the mixed form, the matrix values and
-// the gradient- and direction-side vectors (b, g, phi, beta, p, z, A p) are
+// the gradient- and direction-side vectors (b, g, beta, p, z, A p) are
 // FP32.  The iterate and trial points (x, y, P(y)), the per-node rows and
 // 1/diag stay FP64: the active set is decided on x against the 1e-9 plane
 // tolerance, and the tangent-Jacobi factor s is computed from the FP64
@@ -131,7 +131,7 @@ struct Vecs {
   const T *val;               // SELL values
   const double *dinv;         // 1/diag(A)
   double *x, *y, *py;         // iterate and trial points
-  T *b, *g, *phi, *beta;      // gradient side
+  T *b, *g, *beta;            // gradient side
   T *p, *z, *ap;              // search direction side
   T *p2;                      // second p buffer (mixed inner: p' = z - beta p
                               // is written while neighbours still gather p)

@@ -626,17 +626,26 @@ __device__ __forceinline__ V3 round_to(V3 a) {  // the value a store to T storag
   return V3{(double)(T)a.x, (double)(T)a.y, (double)(T)a.z};
 }
 
+// beta on a node without a row is g - phi = 0, and nothing else reads phi
+// across launches: phi is not stored, and beta only where the node has a row.
+// INIT writes the zeros of the other nodes into both beta buffers, so the
+// gathers of PROP1 find them (28 of a CG step's 158 bytes per node in the
+// mixed form, 48 of 254 in FP64, were these two stores).
+template <class T>
+__device__ __forceinline__ void st_beta(T *beta, const Row &R, int r, V3 be) {
+  if (R.has) st3(beta, r, be);
+}
+
 // computeGradients(g) + proportional (MPRGPSolver.h:163-181) for one row at
-// gradient g (as stored), face f and iterate x: phi and beta stored, the
-// loop head's sums in slots 0-2.
+// gradient g (as stored), face f and iterate x: beta stored, the loop head's
+// sums in slots 0-2.
 template <class T>
 __device__ __forceinline__ void loop_head_row(const Vecs<T> &v, const Row &R, bool f, V3 g, V3 x,
                                               double alpha_bar, int r, double (&P)[kNumPart]) {
   const V3 gs = round_to<T>(g);
   const V3 ph = phi_of(R, f, gs);
   const V3 be = beta_of(R, f, gs, ph);
-  st3(v.phi, r, ph);
-  st3(v.beta, r, be);
+  st_beta(v.beta, R, r, be);
   const V3 gp = add(ph, be);
   P[0] += dot3(gp, gp);
   P[1] += dot3(be, be);
@@ -693,14 +702,17 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       V3 ph = phi_of(R, f, g);
       V3 z = precond_of(v, pre, R, f, r, g, ph);
       st3(v.g, r, g);
-      st3(v.z, r, z);
+      if (st.variant == VAR_CLASSIC) st3(v.z, r, z);  // CG_AP's z is p
       st3(v.p, r, z);
       gmem(q.face)[r] = f;
       if (op == OP_EXP3) st3(yc, r, ld3(v.py, r));
-      // INIT and EXP3 end with the next outer iteration's head (its phi
-      // replaces this one); the classic CL_EXP2 is followed by TOP
-      if (op == OP_CL_EXP2) st3(v.phi, r, ph);
-      else loop_head_row(v, R, f, g, xr, st.alpha_bar, r, P);
+      if (op == OP_INIT && !R.has) {
+        st3(v.beta, r, V3{0.0, 0.0, 0.0});
+        st3(v.beta2, r, V3{0.0, 0.0, 0.0});
+      }
+      // INIT and EXP3 end with the next outer iteration's head; the classic
+      // CL_EXP2 is followed by TOP
+      if (op != OP_CL_EXP2) loop_head_row(v, R, f, g, xr, st.alpha_bar, r, P);
       break;
     }
     case OP_TOP: {
@@ -722,7 +734,8 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       V3 pr = ld3(v.p, r);
       P[0] += dot3(pr, acc[0]);
       const V3 gr = ld3(v.g, r);
-      P[1] += dot3(ld3(v.z, r), gr);
+      // CG_AP runs at the CG entry only, where p = z (:210-215, 232-241)
+      P[1] += dot3(op == OP_CL_AP ? ld3(v.z, r) : pr, gr);
       if (mixed && st.cg_entry) P[2] += dot3(ld3(xc, r), sub(gr, ld3(v.b, r)));
       if (op == OP_CL_AP) {
         // stepLimit (MPRGPProjection.h:263-282)
@@ -797,7 +810,6 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       const V3 ph = phi_of(R, f, g);
       const V3 z = precond_of(v, pre, R, f, r, g, ph);
       st3(v.g, r, g);
-      st3(v.phi, r, ph);
       st3(v.z, r, z);
       // sums over the values later reads of z, g and phi see
       const V3 gs = round_to<T>(g), phs = round_to<T>(ph);
@@ -807,7 +819,7 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       // the other buffer, which only an accepted step makes current (a
       // rejected step's proportioning reads the old beta)
       const V3 be = beta_of(R, f, gs, phs);
-      st3(v.beta2, r, be);
+      st_beta(v.beta2, R, r, be);
       const V3 gp = add(phs, be);
       P[4] += dot3(gp, gp);
       P[5] += dot3(be, be);
@@ -877,12 +889,11 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       const V3 ph = phi_of(R, f, g);
       const V3 z = precond_of(v, pre, R, f, r, g, ph);
       st3(v.g, r, g);
-      st3(v.phi, r, ph);
       st3(v.z, r, z);
       P[2] += dot3(z, ap);
       P[3] += dot3(z, g);
       const V3 be = beta_of(R, f, g, ph);
-      st3(v.beta2, r, be);
+      st_beta(v.beta2, R, r, be);
       const V3 gp = add(ph, be);
       P[4] += dot3(gp, gp);
       P[5] += dot3(be, be);
@@ -902,13 +913,12 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       V3 ph = phi_of(R, f, g);
       V3 z = precond_of(v, pre, R, f, r, g, ph);
       st3(v.g, r, g);
-      st3(v.phi, r, ph);
       st3(v.z, r, z);
       P[0] += dot3(z, ap);
       P[1] += dot3(z, g);  // the next step's alpha numerator
       // computeGradients(g, false) and proportional at the new x
       const V3 be = beta_of(R, f, g, ph);
-      st3(v.beta, r, be);
+      st_beta(v.beta, R, r, be);
       const V3 gp = add(ph, be);
       P[2] += dot3(gp, gp);
       P[3] += dot3(be, be);
@@ -978,7 +988,7 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       V3 z = precond_of(v, pre, R, f, r, g, ph);
       st3(xc, r, xn);
       st3(v.g, r, g);
-      st3(v.z, r, z);
+      if (st.variant == VAR_CLASSIC) st3(v.z, r, z);
       st3(v.p, r, z);
       gmem(q.face)[r] = f;
       loop_head_row(v, R, f, g, xn, st.alpha_bar, r, P);  // the next iteration's head
@@ -994,7 +1004,6 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       V3 ph = phi_of(R, f, g);
       V3 z = precond_of(v, pre, R, f, r, g, ph);
       st3(v.g, r, g);
-      st3(v.phi, r, ph);
       st3(v.z, r, z);
       P[0] += dot3(z, ap);
       break;

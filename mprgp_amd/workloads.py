@@ -74,6 +74,22 @@ _STREAMS = {
     "R_FINAL": ("rows", "x64", "face", "x64"),
 }
 
+# Streams of the list above that the kernels do not move: phi is never stored,
+# beta only on the few nodes with a row (it is zero elsewhere; INIT writes the
+# zeros), and p stands for z where p = z.  ``moved=True`` leaves them out.
+_UNMOVED = {
+    "EXP3": ("phi", "z", "beta"),
+    "CL_EXP2": ("phi",),
+    "TOP": ("phi", "beta"),
+    "INIT": ("phi", "z"),
+    "CG_AP": ("z",),
+    "CG_A": ("phi", "beta"),
+    "CG_PYG": ("phi", "beta"),
+    "CG_YA": ("phi", "beta"),
+    "PROP2": ("phi", "z", "beta"),
+    "CL_CG": ("phi",),
+}
+
 # FP32 streams of the mixed form's inner solve; everything else (x, y, P(y),
 # 1/diag, the rows) is FP64.
 MIXED_F32 = {"M", "b", "g", "phi", "beta", "p", "z", "ap"}
@@ -96,13 +112,17 @@ def spmv_bytes(N, nb, s=8, idx=4):
     return nb * (9 * s + idx) + 4 * (N + 1) + 2 * 3 * N * s
 
 
-def op_bytes(op, N, nb, m, mixed=False, precond=True, idx=4):
+def op_bytes(op, N, nb, m, mixed=False, precond=True, idx=4, moved=False):
     """Algorithmic HBM bytes of one device op on one QP (ideal traffic: every
     stream read or written once).  ``mixed``: the inner-solve ops read the
-    FP32 matrix and FP32 direction vectors; ``idx``: bytes per column index."""
+    FP32 matrix and FP32 direction vectors; ``idx``: bytes per column index;
+    ``moved``: without the streams the kernels leave out (``_UNMOVED``)."""
     name = OPS[op]
     total = 0
-    streams = _STREAMS.get(name, ())
+    streams = list(_STREAMS.get(name, ()))
+    if moved:
+        for st in _UNMOVED.get(name, ()):
+            streams.remove(st)
     for st in streams:
         if st == "rows":
             total += N + 48 * m
@@ -123,10 +143,10 @@ def op_bytes(op, N, nb, m, mixed=False, precond=True, idx=4):
     return total
 
 
-def solve_bytes(counts, N, nb, m, mixed=False, precond=True, idx=4):
+def solve_bytes(counts, N, nb, m, mixed=False, precond=True, idx=4, moved=False):
     """Algorithmic bytes of a whole solve from its per-op launch counts."""
     total = 0
     for op, k in enumerate(counts[:len(OPS)]):
         if k:
-            total += int(k) * op_bytes(op, N, nb, m, mixed, precond, idx)
+            total += int(k) * op_bytes(op, N, nb, m, mixed, precond, idx, moved)
     return total
