@@ -21,7 +21,7 @@
 namespace mprgp {
 
 constexpr int kSlice = 64;       // rows per SELL slice = lanes per wavefront
-constexpr int kNumPart = 8;      // partial sums per tile (most any op produces: 7)
+constexpr int kNumPart = 8;      // partial sums per tile (most any op produces: 8)
 constexpr double kEps = 1e-9;    // ScalarUtil<double>::scalar_eps of the simulator
 constexpr double kDblMax = 1.7976931348623157e308;  // ScalarUtil<double>::scalar_max
 
@@ -34,12 +34,12 @@ enum Op : int {
   OP_INIT,       // g = Ax - b, face(x), phi, z, p = z, and the loop head (TOP)
   OP_TOP,        // loop head: phi, beta, |phi+beta|^2, beta.beta, phitphi
   OP_CG_AP,      // AP = A p, p.AP, z.g
-  OP_CG_PY,      // y = x - alpha p, py = P(y), feasibility of y
-  OP_CG_Y,       // A py (and A x at CG entry): objective values
+  OP_CG_Y,       // FP64 CG entry: y = x - alpha p, feasibility, A P(y) with P(y)
+                 // formed at the gather, A x: objective values
   OP_CG_A,       // (x = y by buffer swap) g -= alpha AP, phi, z, z.AP, z.g,
                  // beta, |phi+beta|^2, beta.beta, phitphi
-  OP_EXP1,       // y = P(x)
-  OP_EXP2,       // g = A y - b, face(y), phi, y' = y - abar phi, x = P(y')
+  OP_EXP2,       // y = P(x), formed at the gather; g = A y - b, face(y), phi,
+                 // y' = y - abar phi, x = P(y') into the other x buffer
   OP_EXP3,       // g = A x - b, face(x), phi, z, p = z, y = y', and the loop head
   OP_PROP1,      // g = A x - b, AD = A beta, beta.AD, g.beta
   OP_PROP2,      // x = P(x - a beta), g -= a AD, face(x), phi, z, p = z, and
@@ -60,8 +60,8 @@ enum Op : int {
                  // |phi+beta|^2, beta.beta, phitphi
   OP_CG_BAP,     // p' = z - beta p into the other p buffer and AP = A p' with
                  // p' formed at the gather from z and p, p'.AP
-  OP_CG_YA,      // FP64, after the first CG step: CG_Y, then CG_A applied
-                 // speculatively (beta into the other beta buffer)
+  OP_CG_YA,      // FP64, after the first CG step: CG_Y without A x, then CG_A
+                 // applied speculatively (beta into the other beta buffer)
   OP_NUM
 };
 
@@ -80,7 +80,7 @@ struct alignas(128) QpState {
   int iteration, num_cg, num_exp, num_prop;
   int max_it;
   int prop;          // result_is_prop
-  int cg_entry;      // next CG_Y also evaluates f(x)
+  int cg_entry;      // the CG loop is being entered: the step evaluates f(x) too
   int y_valid, y_feas;
   int code;
   int active;

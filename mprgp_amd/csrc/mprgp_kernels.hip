@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "mprgp_host.h"
 
@@ -69,11 +70,26 @@ __device__ __forceinline__ void st3(T *v, int r, V3 a) {
 }
 __device__ __forceinline__ V3 add(V3 a, V3 b) { return V3{a.x + b.x, a.y + b.y, a.z + b.z}; }
 __device__ __forceinline__ V3 sub(V3 a, V3 b) { return V3{a.x - b.x, a.y - b.y, a.z - b.z}; }
-// a - s*b
-__device__ __forceinline__ V3 axmy(V3 a, double s, V3 b) {
-  return V3{a.x - s * b.x, a.y - s * b.y, a.z - s * b.z};
+// The per-node functions name their fused multiply-adds, so that a function
+// rounds the same wherever it is inlined: left to the compiler, which of a
+// sum's products is fused depends on how often each is used nearby, and a
+// neighbour's P(y) formed at a gather would differ from its own in the last
+// bit.
+// a + s*b
+__device__ __forceinline__ V3 axpy(V3 a, double s, V3 b) {
+  return V3{__builtin_fma(s, b.x, a.x), __builtin_fma(s, b.y, a.y), __builtin_fma(s, b.z, a.z)};
 }
-__device__ __forceinline__ double dot3(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+// a - s*b
+__device__ __forceinline__ V3 axmy(V3 a, double s, V3 b) { return axpy(a, -s, b); }
+__device__ __forceinline__ double dot3(V3 a, V3 b) {
+  return __builtin_fma(a.z, b.z, __builtin_fma(a.x, b.x, a.y * b.y));
+}
+// P(y).A P(y) at the FP64 CG entry rounds its first product, not its second:
+// the monotone test f(P(y)) <= f(x) decides ties by rounding near the
+// minimum, and this order keeps those decisions where they have been.
+__device__ __forceinline__ double dot3_x(V3 a, V3 b) {
+  return __builtin_fma(a.z, b.z, __builtin_fma(a.y, b.y, a.x * b.x));
+}
 
 // The half-space row of one node (at most one per node).
 struct Row {
@@ -103,7 +119,16 @@ __device__ __forceinline__ V3 proj(const Row &R, V3 x) {
   if (!R.has) return x;
   double v = (R.c - dot3(R.n, x)) / R.jj;
   double lam = (v < 0.0) ? 0.0 : v;
-  return V3{x.x + R.n.x * lam, x.y + R.n.y * lam, x.z + R.n.z * lam};
+  return axpy(x, lam, R.n);
+}
+
+// proj for a node with a row whose division only a violated row runs: at a
+// gather it would be most of the work per neighbour (about 30 of 50 FP64
+// instructions), and few neighbours violate their plane.  lambda = 0
+// otherwise; a NaN takes the division and stays one.
+__device__ __forceinline__ V3 proj_rare(const V3 &n, double c, double jj, V3 x) {
+  const double v = c - dot3(n, x);
+  return !(v <= 0.0) ? axpy(x, v / jj, n) : x;
 }
 
 // DECIDE_FACE (MPRGPProjection.h:283-297): |n.x - c| < eps.
@@ -120,7 +145,7 @@ __device__ __forceinline__ double infeasible(const Row &R, V3 x) {
 __device__ __forceinline__ V3 phi_of(const Row &R, bool face, V3 g) {
   if (!face) return g;
   double lam = -dot3(R.n, g) / R.jj;
-  return V3{g.x + R.n.x * lam, g.y + R.n.y * lam, g.z + R.n.z * lam};
+  return axpy(g, lam, R.n);
 }
 
 // BETA (MPRGPProjection.h:368-383): chopped gradient.  Rows outside the
@@ -133,7 +158,7 @@ __device__ __forceinline__ V3 beta_of(const Row &R, bool face, V3 g, V3 phi) {
     double v = lam / R.jj;
     lam = (0.0 < v) ? v : 0.0;
   }
-  return V3{b.x - R.n.x * lam, b.y - R.n.y * lam, b.z - R.n.z * lam};
+  return axmy(b, lam, R.n);
 }
 
 // DiagonalDecouplePreconSolver::solve (MPRGPPrecondition.h:91-105):
@@ -148,7 +173,7 @@ __device__ __forceinline__ V3 precond_of(const Vecs<T> &v, bool on, const Row &R
   if (face) {
     V3 jm{R.n.x * d.x, R.n.y * d.y, R.n.z * d.z};
     double lam = R.s * dot3(jm, g);
-    z = V3{z.x - jm.x * lam, z.y - jm.y * lam, z.z - jm.z * lam};
+    z = axmy(z, lam, jm);
   }
   return z;
 }
@@ -168,63 +193,130 @@ __device__ __forceinline__ V3 precond_of(const Vecs<T> &v, bool on, const Row &R
 // 4.97 TB/s).  Matrices that fit stay cached from launch to launch instead.
 // C: the column index type, 32-bit or 16-bit (2 of the 40 bytes an FP32
 // block streams: on the 256-QP batch, 3.1% shorter launches).
-template <int NV, int U = (NV == 1 ? 3 : 1), bool NT = false, class C, class T, class G>
-__device__ __forceinline__ void spmv_row(const int *sl_off, const C *col, const T *val, int s, int lane,
-                                         G gather, V3 (&acc)[NV]) {
+// The blocks left after the full rounds of U form one last round: which of
+// its slots exist is the same on every lane (W is the slice's), so all of its
+// loads are in flight together too.
+template <class T>
+__device__ __forceinline__ void block_mul(V3 &acc, const T (&a)[9], V3 x) {
+  acc.x = __builtin_fma((double)a[0], x.x, acc.x);
+  acc.x = __builtin_fma((double)a[1], x.y, acc.x);
+  acc.x = __builtin_fma((double)a[2], x.z, acc.x);
+  acc.y = __builtin_fma((double)a[3], x.x, acc.y);
+  acc.y = __builtin_fma((double)a[4], x.y, acc.y);
+  acc.y = __builtin_fma((double)a[5], x.z, acc.y);
+  acc.z = __builtin_fma((double)a[6], x.x, acc.z);
+  acc.z = __builtin_fma((double)a[7], x.y, acc.z);
+  acc.z = __builtin_fma((double)a[8], x.z, acc.z);
+}
+
+// One round: blocks k .. k+U-1 of the lane's row, or the n < U left ones.
+// gather_all(j, xs, n) loads the input vectors at the round's columns.
+template <int NV, int U, bool NT, bool FULL, class T, class CP, class VP, class G>
+__device__ __forceinline__ void spmv_round(CP cp, VP vp, int k, int n, G &gather_all, V3 (&acc)[NV]) {
+  int j[U];
+  T a[U][9];  // kept in the storage precision until its multiply
+  V3 xs[U][NV];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (!FULL && u >= n) break;
+    j[u] = (int)ldm<NT>(cp + (k + u) * kSlice);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (!FULL && u >= n) break;
+#pragma unroll
+    for (int e = 0; e < 9; ++e) a[u][e] = ldm<NT>(vp + (size_t)(k + u) * (9 * kSlice) + e * kSlice);
+  }
+  gather_all(j, xs, FULL ? U : n);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (!FULL && u >= n) break;
+#pragma unroll
+    for (int t = 0; t < NV; ++t) block_mul(acc[t], a[u], xs[u][t]);
+  }
+}
+
+template <int NV, int U, bool NT, class C, class T, class G>
+__device__ __forceinline__ void spmv_rounds(const int *sl_off, const C *col, const T *val, int s, int lane,
+                                            G gather_all, V3 (&acc)[NV]) {
 #pragma unroll
   for (int t = 0; t < NV; ++t) acc[t] = V3{0.0, 0.0, 0.0};
   const int b0 = gmem(sl_off)[s];
-  const int W = (gmem(sl_off)[s + 1] - b0) / kSlice;
+  const int W = __builtin_amdgcn_readfirstlane((gmem(sl_off)[s + 1] - b0) / kSlice);
   const auto *cp = gmem(col) + b0 + lane;
   const auto *vp = gmem(val) + (size_t)b0 * 9 + lane;
   int k = 0;
-  for (; k + U <= W; k += U) {
-    int j[U];
-    T a[U][9];  // kept in the storage precision until its multiply
-    V3 xs[U][NV];
+  for (; k + U <= W; k += U) spmv_round<NV, U, NT, true, T>(cp, vp, k, U, gather_all, acc);
+  if (U > 1 && k < W) spmv_round<NV, U, NT, false, T>(cp, vp, k, W - k, gather_all, acc);
+}
+
+template <int NV, int U = (NV == 1 ? 3 : 1), bool NT = false, class C, class T, class G>
+__device__ __forceinline__ void spmv_row(const int *sl_off, const C *col, const T *val, int s, int lane,
+                                         G gather, V3 (&acc)[NV]) {
+  spmv_rounds<NV, U, NT>(
+      sl_off, col, val, s, lane,
+      [&](int (&j)[U], V3 (&xs)[U][NV], int n) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) j[u] = (int)ldm<NT>(cp + (k + u) * kSlice);
+        for (int u = 0; u < U; ++u) {
+          if (u >= n) break;
+          gather(j[u], xs[u]);
+        }
+      },
+      acc);
+}
+
+// The projected gathers hold x, p and the row data of every block in flight:
+// two blocks where the one-vector SpMV takes three, four where it takes six,
+// keep the kernel without spills.
+constexpr int proj_unroll(int ub) { return ub > 3 ? 4 : 2; }
+
+// A P(w) for w = x - alpha p (STEP) or w = x, with w and its projection
+// formed at the gather from the neighbours' x, p and rows, none of which the
+// launch writes; NV = 2 also gives A x.  A round first loads its columns' x,
+// p and row flags, then, on the lanes that have a flagged column, all of the
+// round's row data at once (loading every column's row data with the first
+// loads measured the same, also where every node has a row).  Forming P(w) here replaces an elementwise launch
+// before the product.
+template <int NV, int U, bool NT, bool STEP, class C, class T>
+__device__ __forceinline__ void spmv_proj(const QpDev &q, const Vecs<T> &v, const C *col, const double *x,
+                                          double alpha, int s, int lane, V3 (&acc)[NV]) {
+  spmv_rounds<NV, U, NT>(
+      q.sl_off, col, v.val, s, lane,
+      [&](int (&j)[U], V3 (&xs)[U][NV], int n) {
+        unsigned char f[U];
+        V3 pj[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
+          if (u >= n) break;
+          f[u] = gmem(q.cf)[j[u]];
+          xs[u][NV - 1] = ld3(x, j[u]);
+          if (STEP) pj[u] = ld3(v.p, j[u]);
+        }
+        bool any = false;
 #pragma unroll
-      for (int e = 0; e < 9; ++e) a[u][e] = ldm<NT>(vp + (size_t)(k + u) * (9 * kSlice) + e * kSlice);
+        for (int u = 0; u < U; ++u) {
+          if (u >= n) break;
+          any |= f[u] != 0;
+          xs[u][0] = STEP ? axmy(xs[u][NV - 1], alpha, pj[u]) : xs[u][NV - 1];
+        }
+        if (any) {
+          V3 nj[U];
+          double cj[U], jj[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) gather(j[u], xs[u]);
+          for (int u = 0; u < U; ++u) {
+            if (u >= n) break;
+            nj[u] = ld3(v.cn, j[u]);
+            cj[u] = gmem(v.cc)[j[u]];
+            jj[u] = gmem(v.cj)[j[u]];
+          }
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int t = 0; t < NV; ++t) {
-        acc[t].x += (double)a[u][0] * xs[u][t].x;
-        acc[t].x += (double)a[u][1] * xs[u][t].y;
-        acc[t].x += (double)a[u][2] * xs[u][t].z;
-        acc[t].y += (double)a[u][3] * xs[u][t].x;
-        acc[t].y += (double)a[u][4] * xs[u][t].y;
-        acc[t].y += (double)a[u][5] * xs[u][t].z;
-        acc[t].z += (double)a[u][6] * xs[u][t].x;
-        acc[t].z += (double)a[u][7] * xs[u][t].y;
-        acc[t].z += (double)a[u][8] * xs[u][t].z;
-      }
-  }
-  for (; k < W; ++k) {
-    const int j = (int)ldm<NT>(cp + k * kSlice);
-    T a[9];
-#pragma unroll
-    for (int e = 0; e < 9; ++e) a[e] = ldm<NT>(vp + (size_t)k * (9 * kSlice) + e * kSlice);
-    V3 xs[NV];
-    gather(j, xs);
-#pragma unroll
-    for (int t = 0; t < NV; ++t) {
-      acc[t].x += (double)a[0] * xs[t].x;
-      acc[t].x += (double)a[1] * xs[t].y;
-      acc[t].x += (double)a[2] * xs[t].z;
-      acc[t].y += (double)a[3] * xs[t].x;
-      acc[t].y += (double)a[4] * xs[t].y;
-      acc[t].y += (double)a[5] * xs[t].z;
-      acc[t].z += (double)a[6] * xs[t].x;
-      acc[t].z += (double)a[7] * xs[t].y;
-      acc[t].z += (double)a[8] * xs[t].z;
-    }
-  }
+          for (int u = 0; u < U; ++u) {
+            if (u >= n) break;
+            if (f[u]) xs[u][0] = proj_rare(nj[u], cj[u], jj[u], xs[u][0]);
+          }
+        }
+      },
+      acc);
 }
 
 // ----------------------------------------------------------- reductions
@@ -270,19 +362,15 @@ __device__ __forceinline__ double wave_min(double v) {
 constexpr int kMinSlot = 3;
 __device__ __forceinline__ int sum_slots(int op) {
   switch (op) {
-    case OP_CG_PYG:
+    case OP_CG_PYG: case OP_CG_YA:
       return 8;
-    case OP_CG_YA:
-      return 7;
-    case OP_CG_A:
+    case OP_CG_Y: case OP_CG_A:
       return 5;
     case OP_TOP: case OP_CG_AP: case OP_INIT: case OP_EXP3: case OP_PROP2:
       return 3;
-    case OP_CG_Y:
-      return 4;
     case OP_CL_AP: case OP_PROP1: case OP_CL_PROP1: case OP_POW_IT:
       return 2;
-    case OP_CG_PY: case OP_EXP2: case OP_FINAL: case OP_CL_CG: case OP_CG_BAP:
+    case OP_EXP2: case OP_FINAL: case OP_CL_CG: case OP_CG_BAP:
     case OP_R_START: case OP_R_FINAL:
       return 1;
     default:
@@ -356,7 +444,7 @@ __device__ __forceinline__ void cg_decide(QpState &st, double fnew, double fx_en
   } else if (st.residual <= st.tol) {
     st.op = OP_FINAL;
   } else {
-    st.op = (st.prop || !st.y_valid || !st.y_feas) ? OP_EXP1 : OP_PROP1;
+    st.op = (st.prop || !st.y_valid || !st.y_feas) ? OP_EXP2 : OP_PROP1;
   }
 }
 
@@ -384,7 +472,7 @@ __device__ __forceinline__ void loop_head(QpState &st, const Sums &S) {
     st.cg_entry = 1;
     st.op = OP_CG_AP;
   } else {
-    st.op = (!st.y_valid || !st.y_feas) ? OP_EXP1 : OP_PROP1;
+    st.op = (!st.y_valid || !st.y_feas) ? OP_EXP2 : OP_PROP1;
   }
 }
 
@@ -449,13 +537,8 @@ __device__ void control(QpState &st, const Sums &S) {
       st.zg = S.v[1];
       st.alpha = st.zg / st.pd;
       if (st.mixed && st.cg_entry) st.fx_entry = 0.5 * S.v[2];  // f(x) = x'(g - b)/2, g = A x - b
-      st.op = st.mixed ? OP_CG_PYG : OP_CG_PY;
-      break;
-    case OP_CG_PY:
-      st.y_valid = 1;
-      st.y_feas = S.v[0] == 0.0;
-      // the CG entry needs f(x) too (four sums): its step takes CG_Y, CG_A
-      st.op = st.cg_entry ? OP_CG_Y : OP_CG_YA;
+      // the CG entry needs f(x) too (four sums): its FP64 step takes CG_Y, CG_A
+      st.op = st.mixed ? OP_CG_PYG : OP_CG_Y;
       break;
     case OP_CG_PYG: {
       // mixed inner solve: f(y) = f(x) - alpha p'g + alpha^2 p'Ap/2 and
@@ -477,9 +560,13 @@ __device__ void control(QpState &st, const Sums &S) {
       break;
     }
     case OP_CG_Y:
+      st.y_valid = 1;
+      st.y_feas = S.v[4] == 0.0;
       cg_decide(st, 0.5 * S.v[0] - S.v[1], 0.5 * S.v[2] - S.v[3], false);
       break;
     case OP_CG_YA:
+      st.y_valid = 1;
+      st.y_feas = S.v[7] == 0.0;
       st.zap = S.v[2];
       st.zg = S.v[3];  // z.g after the update: the next step's alpha numerator
       st.res_next = sqrt(S.v[4]);
@@ -497,12 +584,10 @@ __device__ void control(QpState &st, const Sums &S) {
       st.pb ^= 1;  // p' went to the other buffer
       st.pd = S.v[0];
       st.alpha = st.zg / st.pd;
-      st.op = st.mixed ? OP_CG_PYG : OP_CG_PY;
-      break;
-    case OP_EXP1:
-      st.op = OP_EXP2;
+      st.op = st.mixed ? OP_CG_PYG : OP_CG_YA;
       break;
     case OP_EXP2:
+      st.xb ^= 1;  // the new x went to the other buffer
       st.y_valid = 1;
       st.y_feas = S.v[0] == 0.0;
       st.op = OP_EXP3;
@@ -750,20 +835,11 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       }
       break;
     }
-    case OP_CG_PY: {
-      const V3 xr = ld3(xc, r), pr = ld3(v.p, r);  // in flight with the row flag
-      Row R = ldrow(q, v, r);
-      V3 y = axmy(xr, st.alpha, pr);
-      st3(yc, r, y);
-      st3(v.py, r, proj(R, y));
-      P[0] += infeasible(R, y);
-      break;
-    }
     case OP_CG_PYG: {
       // Mixed inner solve, CGMonotonicStep (MPRGPSolver.h:281-297) in one
       // pass: the trial point with the sums for f(y), and the gradient
       // update of an accepted step applied in place.  A rejected step leaves
-      // the CG loop through EXP1/EXP2, PROP1 or FINAL, and the first two
+      // the CG loop through EXP2, PROP1 or FINAL, and the first two
       // recompute g = A x - b, phi and z before reading them (the reference
       // does the same: MPRGPSolver.h:255-261, 435-437); FINAL reads x only.
       // The face stays fixed inside the CG loop.
@@ -846,45 +922,44 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       break;
     }
     case OP_CG_Y: {
-      const double *py = v.py;
-      V3 pyr = ld3(v.py, r);
-      V3 br = ld3(v.b, r);
-      if (st.cg_entry) {
-        const double *x = xc;
+      // the CG entry: y = x - alpha p, f(P(y)) and f(x)  (MPRGPSolver.h:276-284)
+      if constexpr (std::is_same_v<T, double>) {
         V3 acc[2];
-        spmv_row<2, 1, NT>(q.sl_off, cols<C16>(q), v.val, s, lane, [&](int j, V3 (&xs)[2]) {
-          xs[0] = ld3(py, j);
-          xs[1] = ld3(x, j);
-        }, acc);
-        V3 xr = ld3(xc, r);
-        P[0] += dot3(pyr, acc[0]);
+        spmv_proj<2, UB / 3, NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
+        const V3 xr = ld3(xc, r), pr = ld3(v.p, r);  // in flight with the row flag
+        Row R = ldrow(q, v, r);
+        const V3 y = axmy(xr, st.alpha, pr);
+        st3(yc, r, y);
+        const V3 pyr = proj(R, y), br = ld3(v.b, r);
+        P[0] += dot3_x(pyr, acc[0]);
         P[1] += dot3(pyr, br);
         P[2] += dot3(xr, acc[1]);
         P[3] += dot3(xr, br);
-      } else {
-        V3 acc[1];
-        spmv_row<1, UB, NT>(q.sl_off, cols<C16>(q), v.val, s, lane, [&](int j, V3 (&xs)[1]) { xs[0] = ld3(py, j); }, acc);
-        P[0] += dot3(pyr, acc[0]);
-        P[1] += dot3(pyr, br);
+        P[4] += infeasible(R, y);
       }
       break;
     }
     case OP_CG_YA: {
-      // CGMonotonicStep (MPRGPSolver.h:283-302) after the CG entry: f(P(y))
-      // by A P(y) as CG_Y, then CG_A's update applied speculatively at x = y.
-      // A rejected step leaves the CG loop through EXP1/EXP2, PROP1 or FINAL,
-      // and the first two recompute g, phi and z before reading them
+      // CGMonotonicStep (MPRGPSolver.h:281-302) after the CG entry: the trial
+      // point y = x - alpha p and its feasibility, f(P(y)) by A P(y) with
+      // P(y) formed at the gather, then CG_A's update applied speculatively at
+      // x = y.  A rejected step leaves the CG loop through EXP2, PROP1 or
+      // FINAL, and the first two recompute g and z before reading them
       // (MPRGPSolver.h:255-261, 435-437); FINAL reads x only; beta goes to
       // the other buffer, current only once the step is accepted.
-      const double *py = v.py;
+      if constexpr (!std::is_same_v<T, double>) break;
       V3 acc[1];
-      spmv_row<1, UB, NT>(q.sl_off, cols<C16>(q), v.val, s, lane, [&](int j, V3 (&xs)[1]) { xs[0] = ld3(py, j); }, acc);
-      const V3 pyr = ld3(v.py, r);
-      P[0] += dot3(pyr, acc[0]);
-      P[1] += dot3(pyr, ld3(v.b, r));
+      spmv_proj<1, proj_unroll(UB), NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
+      const V3 xr = ld3(xc, r), pr = ld3(v.p, r);
       const bool f = gmem(q.face)[r];  // in flight with the row flag
       const V3 ap = ld3(v.ap, r), gr = ld3(v.g, r);
       Row R = ldrow(q, v, r);
+      const V3 y = axmy(xr, st.alpha, pr);
+      st3(yc, r, y);
+      const V3 pyr = proj(R, y);
+      P[0] += dot3(pyr, acc[0]);
+      P[1] += dot3(pyr, ld3(v.b, r));
+      P[7] += infeasible(R, y);
       const V3 g = axmy(gr, st.alpha, ap);
       const V3 ph = phi_of(R, f, g);
       const V3 z = precond_of(v, pre, R, f, r, g, ph);
@@ -897,7 +972,6 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       const V3 gp = add(ph, be);
       P[4] += dot3(gp, gp);
       P[5] += dot3(be, be);
-      const V3 y = ld3(yc, r);
       const V3 px = proj(R, axmy(y, st.alpha_bar, ph));
       P[6] += dot3(sub(y, px), ph);
       break;
@@ -927,27 +1001,22 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       P[4] += dot3(sub(x, px), ph);
       break;
     }
-    case OP_EXP1: {
-      Row R = ldrow(q, v, r);
-      st3(yc, r, proj(R, ld3(xc, r)));
-      break;
-    }
     case OP_EXP2: {
-      // ExpMonotonicStep, first half (MPRGPSolver.h:255-261): the new y goes
-      // to py because neighbours still gather y in this launch.
+      // ExpMonotonicStep, first half (MPRGPSolver.h:250-261) with y = P(x)
+      // formed at the gather.  Neighbours gather x in this launch, so the new
+      // x goes to the other buffer (y's; the control swaps them) and the new
+      // y to py.
       V3 acc[1];
-      const double *y = yc;
-      spmv_row<1, UB, NT>(q.sl_off, cols<C16>(q), v.val, s, lane, [&](int j, V3 (&xs)[1]) { xs[0] = ld3(y, j); }, acc);
+      spmv_proj<1, proj_unroll(UB), NT, false>(q, v, cols<C16>(q), xc, 0.0, s, lane, acc);
       V3 g = sub(acc[0], ld3(v.b, r));
+      const V3 xr = ld3(xc, r);  // in flight with the row flag
       Row R = ldrow(q, v, r);
-      V3 yr = ld3(yc, r);
+      V3 yr = proj(R, xr);
       bool f = face_of(R, yr);
       V3 ph = phi_of(R, f, g);
       V3 yn = axmy(yr, st.alpha_bar, ph);
-      st3(v.g, r, g);
       st3(v.py, r, yn);
-      st3(xc, r, proj(R, yn));
-      gmem(q.face)[r] = f;
+      st3(yc, r, proj(R, yn));
       P[0] += infeasible(R, yn);
       break;
     }

@@ -14,8 +14,8 @@ import mprgp_amd as M
 from mprgp_amd import problems
 
 # op indices of the device state machine (mprgp_dev.h)
-OPS = ["DONE", "PROJX", "POW_IT", "POW_SAVE", "INIT", "TOP", "CG_AP", "CG_PY", "CG_Y",
-       "CG_A", "EXP1", "EXP2", "EXP3", "PROP1", "PROP2", "FINAL", "CL_AP", "CL_CG",
+OPS = ["DONE", "PROJX", "POW_IT", "POW_SAVE", "INIT", "TOP", "CG_AP", "CG_Y",
+       "CG_A", "EXP2", "EXP3", "PROP1", "PROP2", "FINAL", "CL_AP", "CL_CG",
        "CL_EXP", "CL_EXP2", "CL_PROP1", "R_START", "R_UPD", "R_FINAL", "CG_PYG",
        "CG_BAP", "CG_YA"]
 
@@ -55,14 +55,12 @@ _STREAMS = {
     "TOP": ("rows", "face", "g", "x", "phi", "beta"),
     "CG_AP": ("M", "p", "ap", "z", "g"),
     "CL_AP": ("M", "p", "ap", "z", "g", "rows", "x"),
-    "CG_PY": ("rows", "x", "p", "y", "py"),
-    "CG_Y": ("M", "py", "b"),
+    "CG_Y": ("M", "x", "p", "y", "b", "rows"),
     "CG_A": ("rows", "face", "ap", "g", "dinv", "x", "g", "phi", "z", "beta"),
     "CG_PYG": ("rows", "face", "x", "p", "y", "g", "ap", "dinv", "g", "phi", "z", "beta"),
     "CG_BAP": ("M", "z", "p", "p", "ap"),
-    "CG_YA": ("M", "py", "b", "rows", "face", "ap", "g", "dinv", "y", "g", "phi", "z", "beta"),
-    "EXP1": ("rows", "x", "y"),
-    "EXP2": ("M", "y", "b", "rows", "g", "py", "x", "face"),
+    "CG_YA": ("M", "x", "p", "y", "b", "rows", "face", "ap", "g", "dinv", "g", "phi", "z", "beta"),
+    "EXP2": ("M", "x", "b", "rows", "py", "x"),
     "PROP1": ("M", "x", "beta", "b", "g", "ap"),
     "PROP2": ("rows", "x", "beta", "g", "ap", "dinv", "x", "g", "phi", "z", "p", "face", "beta"),
     "FINAL": ("rows", "x", "face", "x"),
