@@ -186,7 +186,7 @@ struct ProjArgs {
 // through the QP table.
 struct Tile {
   QpState *st;   // the QP's st[0], st[1] (launch parity)
-  double *part;  // the QP's [2][kNumPart][nt] partial sums (launch parity, slot-major)
+  double *part;  // the QP's [2][nt][kNumPart] partial sums (launch parity, tile-major)
   int qp;        // index into the batch's QpDev table
   int slice0;
   int slices;

@@ -339,23 +339,87 @@ __device__ __forceinline__ double lane_value(double v, int l) {
                           __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
+// The two operands of a sum over row pairs: v_permlane16_swap of v with
+// itself gives rows {0, 0, 2, 2} and {1, 1, 3, 3}, v_permlane32_swap the lower
+// and the upper half in both halves.
+typedef unsigned int U2 __attribute__((ext_vector_type(2)));
+template <bool HALVES>
+__device__ __forceinline__ void row_pair(double v, double &a, double &b) {
+  const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+  U2 l, h;
+  if constexpr (HALVES) {
+    l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  } else {
+    l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  }
+  a = __hiloint2double((int)h[0], (int)l[0]);
+  b = __hiloint2double((int)h[1], (int)l[1]);
+}
+
 // Sum over the wavefront in a fixed order (pairs, quads, eighths, rows of
 // 16, then the four rows), the same value in every lane: each combining
 // step adds the same two operands in both lanes of a partner pair.
+__device__ __forceinline__ double sum_rows(double v) {  // of the rows' totals
+  double a, b;
+  row_pair<false>(v, a, b);
+  row_pair<true>(a + b, a, b);
+  return a + b;
+}
 __device__ __forceinline__ double wave_sum(double v) {
   v += dpp<kDppSwap1>(v);
   v += dpp<kDppSwap2>(v);
   v += dpp<kDppHalfMirror>(v);
   v += dpp<kDppMirror>(v);
-  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+  return sum_rows(v);
 }
 __device__ __forceinline__ double wave_min(double v) {
   v = fmin(v, dpp<kDppSwap1>(v));
   v = fmin(v, dpp<kDppSwap2>(v));
   v = fmin(v, dpp<kDppHalfMirror>(v));
   v = fmin(v, dpp<kDppMirror>(v));
-  return fmin(fmin(lane_value(v, 0), lane_value(v, 16)), fmin(lane_value(v, 32), lane_value(v, 48)));
+  double a, b;
+  row_pair<false>(v, a, b);
+  row_pair<true>(fmin(a, b), a, b);
+  return fmin(a, b);
 }
+
+// Several sums over the wavefront at once, each added in wave_sum's order:
+// lane l returns the total of P[sum_slot(l)].  A combining step first halves
+// the number of values a lane holds: of two values it keeps one, sends its
+// partner the other, and adds what it receives.  Which one it keeps follows
+// lane bits that the later steps' partners share (sum_slot), so eight sums
+// take about 60 instructions instead of eight times 37: a lone wavefront
+// issues one instruction every 4-5 cycles, and the sums of the prologue and
+// of the tile's end were 40% of the instructions of a CG launch.
+__device__ __forceinline__ int sum_slot(int lane) {
+  const int b2 = (lane >> 2) & 1;
+  return ((lane ^ b2) & 1) | ((lane ^ (b2 << 1)) & 2) | (((lane >> 2) ^ (lane >> 3)) & 1) << 2;
+}
+template <int kCtrl>
+__device__ __forceinline__ double keep_one(double a, double b, bool second) {
+  return (second ? b : a) + dpp<kCtrl>(second ? a : b);
+}
+template <int N>
+__device__ __forceinline__ double wave_sums(const double *P, int lane) {
+  static_assert(N == 4 || N == 8, "four or eight sums");
+  const int k = sum_slot(lane);
+  double v = keep_one<kDppSwap2>(keep_one<kDppSwap1>(P[0], P[1], k & 1), keep_one<kDppSwap1>(P[2], P[3], k & 1),
+                                 k & 2);
+  if constexpr (N == 8) {
+    const double w = keep_one<kDppSwap2>(keep_one<kDppSwap1>(P[4], P[5], k & 1),
+                                         keep_one<kDppSwap1>(P[6], P[7], k & 1), k & 2);
+    v = keep_one<kDppHalfMirror>(v, w, k & 4);
+  } else {
+    v += dpp<kDppHalfMirror>(v);
+  }
+  v += dpp<kDppMirror>(v);
+  return sum_rows(v);
+}
+// The lane among the first eight that holds slot j's total (wave_sums<4>:
+// the first four lanes; lanes 4-7 hold them again).
+constexpr int slot_lane(int j) { return j < 4 ? j : 11 - j; }
 
 // Partial sums an op produces: slots 0..n-1 reduce with sum.  The classic
 // step-length search (CL_AP) also reduces slot 3 with min.
@@ -1232,39 +1296,43 @@ __device__ void tile_work(const QpDev &q, const Tile &t, int op, const QpState &
   }
 }
 
-// Partial sums of one QP's tiles, slots J0..J0+kGroup-1, summed per lane:
-// every load of a lane's first two columns is issued before the first use.
+// Partial sums of one QP's tiles, slots J0..J0+kGroup-1, summed per lane: lane
+// l adds the tiles l, l + 64, ... in order.  A tile's eight slots are
+// contiguous (64 bytes of its own), so a lane reads them with wide loads and
+// every load of its first two tiles is issued before the first use.
 constexpr int kGroup = 4;
+template <int J0>
+__device__ __forceinline__ void ld_group(const double *pp, int k, double (&a)[kGroup]) {
+  const auto *p = gmem(pp) + (size_t)k * kNumPart + J0;
+#pragma unroll
+  for (int j = 0; j < kGroup; ++j) a[j] = p[j];
+}
 template <int J0>
 __device__ __forceinline__ void sum_part(const double *pp, int nt, int lane, double (&acc)[kNumPart],
                                          double &mn) {
-  double a[2][kGroup];
+  double a[kGroup], b[kGroup];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int k = lane + u * kSlice;
+  for (int j = 0; j < kGroup; ++j) a[j] = b[j] = 0.0;
+  if (lane < nt) ld_group<J0>(pp, lane, a);
+  if (nt > kSlice && lane + kSlice < nt) ld_group<J0>(pp, lane + kSlice, b);
 #pragma unroll
-    for (int j = 0; j < kGroup; ++j) a[u][j] = (k < nt) ? gmem(pp)[(size_t)(J0 + j) * nt + k] : 0.0;
-  }
-#pragma unroll
-  for (int j = 0; j < kGroup; ++j) acc[J0 + j] = a[0][j] + a[1][j];
+  for (int j = 0; j < kGroup; ++j) acc[J0 + j] = a[j] + b[j];
   if (J0 == 0) {
 #pragma unroll
     for (int j = kGroup; j < kNumPart; ++j) acc[j] = 0.0;
-    mn = fmin(lane < nt ? a[0][kMinSlot] : kDblMax, lane + kSlice < nt ? a[1][kMinSlot] : kDblMax);
+    mn = fmin(lane < nt ? a[kMinSlot] : kDblMax, lane + kSlice < nt ? b[kMinSlot] : kDblMax);
   }
-  // QPs of more than 128 tiles: rounds of four columns per lane, every load
-  // of a round issued before its sums, then one last round of the columns
-  // left.  Which columns a round holds is the same on every lane (a column of
-  // 64 tiles exists if its first tile does); in the last round lanes past the
-  // last tile load that tile and do not add it.  Each lane adds its columns
+  // QPs of more than 128 tiles: rounds of four tiles per lane, every load
+  // of a round issued before its sums, then one last round of the tiles
+  // left.  Which columns of 64 tiles a round holds is the same on every lane
+  // (a column exists if its first tile does); in the last round lanes past
+  // the last tile load that tile and do not add it.  Each lane adds its tiles
   // in order, as one column at a time would.
   int k0 = 2 * kSlice;
   for (; k0 + 4 * kSlice <= nt; k0 += 4 * kSlice) {
     double v[4][kGroup];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int j = 0; j < kGroup; ++j) v[u][j] = gmem(pp)[(size_t)(J0 + j) * nt + k0 + u * kSlice + lane];
+    for (int u = 0; u < 4; ++u) ld_group<J0>(pp, k0 + u * kSlice + lane, v[u]);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -1278,9 +1346,7 @@ __device__ __forceinline__ void sum_part(const double *pp, int nt, int lane, dou
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       if (k0 + u * kSlice >= nt) break;
-      const int k = min(k0 + u * kSlice + lane, nt - 1);
-#pragma unroll
-      for (int j = 0; j < kGroup; ++j) v[u][j] = gmem(pp)[(size_t)(J0 + j) * nt + k];
+      ld_group<J0>(pp, min(k0 + u * kSlice + lane, nt - 1), v[u]);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -1322,7 +1388,7 @@ __global__ void __launch_bounds__(TS * kSlice, UB == kUnroll ? MPRGP_STEP_MIN_WA
     mprgp_step(const QpDev *__restrict__ qps,
                                                            const Tile *__restrict__ tiles,
                                                            int *running, int parity) {
-  __shared__ double red[TS][kNumPart];
+  __shared__ double red[TS > 1 ? TS : 1][kNumPart];
   __shared__ QpState sst;
   const int wave = threadIdx.x / kSlice;
   const int lane = threadIdx.x % kSlice;
@@ -1333,7 +1399,7 @@ __global__ void __launch_bounds__(TS * kSlice, UB == kUnroll ? MPRGP_STEP_MIN_WA
   const QpDev &q = qps[t.qp];
   // 1. state the previous launch executed + its partials -> this launch's op.
   //    Wave 0 issues every load (one 8-byte state word per lane, the
-  //    partials slot-major: [parity][slot][tile]) before the first wait.
+  //    partials [parity][tile][slot]) before the first wait.
   if (wave == 0) {
     const StateWord w = gmem(reinterpret_cast<const StateWord *>(t.st + (parity ^ 1)))[lane];
     const int nt = t.nt;
@@ -1347,8 +1413,21 @@ __global__ void __launch_bounds__(TS * kSlice, UB == kUnroll ? MPRGP_STEP_MIN_WA
     const int ns = sum_slots(prev);
     if (ns > kGroup) sum_part<kGroup>(pp, nt, lane, acc, mn);  // the wide ops' upper slots
     Sums S;
+    if (ns > kGroup) {
+      const double tot = wave_sums<8>(acc, lane);
 #pragma unroll
-    for (int j = 0; j < kNumPart; ++j) S.v[j] = (j < ns) ? wave_sum(acc[j]) : 0.0;
+      for (int j = 0; j < kNumPart; ++j) S.v[j] = lane_value(tot, slot_lane(j));
+    } else {
+#pragma unroll
+      for (int j = 0; j < kNumPart; ++j) S.v[j] = 0.0;
+      if (ns > 1) {
+        const double tot = wave_sums<4>(acc, lane);
+#pragma unroll
+        for (int j = 0; j < kGroup; ++j) S.v[j] = lane_value(tot, slot_lane(j));
+      } else if (ns == 1) {
+        S.v[0] = lane_value(wave_sum(acc[0]), 0);
+      }
+    }
     if (prev == OP_CL_AP) S.v[kMinSlot] = wave_min(mn);
     __builtin_amdgcn_wave_barrier();
     if (lane == 0) {
@@ -1377,23 +1456,27 @@ __global__ void __launch_bounds__(TS * kSlice, UB == kUnroll ? MPRGP_STEP_MIN_WA
     for (int j = 0; j < kNumPart; ++j) P[j] = 0.0;
     if (has_min) P[kMinSlot] = kDblMax;
     tile_work<TS, MX, UB, NT, SPW, C16>(q, t, op, st, P);
-    // wave then block reduction in a fixed order, over the op's slots only
+    // wave then block reduction in a fixed order: the first lanes of a wave
+    // hold the slots' totals (slot k), the tile's 64 bytes are written at once
     const int ns = has_min ? kMinSlot + 1 : sum_slots(op);
     if (ns > 0) {
-#pragma unroll
-      for (int j = 0; j < kNumPart; ++j)
-        if (j < ns) P[j] = (has_min && j == kMinSlot) ? wave_min(P[j]) : wave_sum(P[j]);
-      if (lane == 0) {
-#pragma unroll
-        for (int j = 0; j < kNumPart; ++j) red[wave][j] = P[j];
+      const int k = ns == 1 ? lane : sum_slot(lane);
+      double tot = ns == 1 ? wave_sum(P[0]) : (ns <= 4 ? wave_sums<4>(P, lane) : wave_sums<8>(P, lane));
+      if (has_min) {
+        const double mn = wave_min(P[kMinSlot]);
+        if (k == kMinSlot) tot = mn;
       }
-      __syncthreads();
-      if (wave == 0 && lane < ns) {
-        const int j = lane;
-        const bool m = has_min && j == kMinSlot;
-        double acc = red[0][j];
-        for (int w = 1; w < TS; ++w) acc = m ? fmin(acc, red[w][j]) : acc + red[w][j];
-        gmem(t.part)[((size_t)parity * kNumPart + j) * t.nt + t.local] = acc;
+      if constexpr (TS > 1) {
+        if (lane < kNumPart) red[wave][k] = tot;
+        __syncthreads();
+        if (wave == 0 && lane < ns) {
+          const bool m = has_min && lane == kMinSlot;
+          double acc = red[0][lane];
+          for (int w = 1; w < TS; ++w) acc = m ? fmin(acc, red[w][lane]) : acc + red[w][lane];
+          gmem(t.part)[((size_t)parity * t.nt + t.local) * kNumPart + lane] = acc;
+        }
+      } else {
+        if (lane < kNumPart && k < ns) gmem(t.part)[((size_t)parity * t.nt + t.local) * kNumPart + k] = tot;
       }
     }
   }
