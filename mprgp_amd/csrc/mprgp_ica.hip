@@ -16,8 +16,8 @@
 // The sweep is sequential in the user's node order, and it stays so: nodes
 // are grouped into dependency levels (a node's level is one more than the
 // highest level among the nodes it couples to that come before it), and one
-// workgroup runs the levels in order with a barrier between them.  Every
-// node then sees exactly the new and old values the sequential sweep gives
+// workgroup runs the levels in order with a barrier between them, x in an
+// LDS ring where the levels' reach allows (ica_sweep_ring).  Every node then sees exactly the new and old values the sequential sweep gives
 // it, so the sweep is the reference's, not a multicolour variant with other
 // iterates.  Each row adds its terms in the order of its blocks (the input's
 // column order), singly rounded, as the oracle does.
@@ -74,6 +74,15 @@ __global__ void __launch_bounds__(256) ica_dinv(const int *sl_off, const int *co
   inv3(D, dinv + 9 * (size_t)i);
 }
 
+// Cross-lane: the value of the quad's lane kLane.
+template <int kLane>
+__device__ __forceinline__ double quad_lane(double v) {
+  constexpr int ctrl = kLane | kLane << 2 | kLane << 4 | kLane << 6;
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
 // One pass over each row's blocks (internal node order, 3 values per node):
 //   kOffDiag:  out = Da^-1 (sum over blocks off the node of A x  -  b)
 //   kUpper:    out = (jtl - sum over blocks after the node of A x) + b
@@ -81,7 +90,7 @@ __global__ void __launch_bounds__(256) ica_dinv(const int *sl_off, const int *co
 __global__ void __launch_bounds__(256) ica_rows(const int *sl_off, const int *col, const double *val,
                                                 const int *perm, const double *x, const double *b,
                                                 const double *jtl, const double *dinv, double *out, int n_nodes,
-                                                int mode) {
+                                                int mode, const int *pos) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_nodes) return;
   const int s = i / kSlice, l = i % kSlice;
@@ -112,9 +121,10 @@ __global__ void __launch_bounds__(256) ica_rows(const int *sl_off, const int *co
     out[r + 1] = D[3] * t0 + D[4] * t1 + D[5] * t2;
     out[r + 2] = D[6] * t0 + D[7] * t1 + D[8] * t2;
   } else if (mode == kUpper) {
-    out[r] = (jtl[r] - a0) + b[r];
-    out[r + 1] = (jtl[r + 1] - a1) + b[r + 1];
-    out[r + 2] = (jtl[r + 2] - a2) + b[r + 2];
+    double *o = out + 3 * (size_t)(pos ? pos[i] : i);  // pos: the sweep's order
+    o[0] = (jtl[r] - a0) + b[r];
+    o[1] = (jtl[r + 1] - a1) + b[r + 1];
+    o[2] = (jtl[r + 2] - a2) + b[r + 2];
   } else {
     out[r] = (a0 - b[r]) - jtl[r];
     out[r + 1] = (a1 - b[r + 1]) - jtl[r + 1];
@@ -191,6 +201,168 @@ __global__ void __launch_bounds__(512) ica_sweep(const double *lo_val, const int
 }
 
 constexpr int kSweepThreads = 512;
+
+// The same sweep with x kept in the LDS.  The sweep is one CU's work and was
+// bound by each level's chain: level bounds, node and block range, columns,
+// x, products, the store of x and its acknowledgement before the barrier.
+// Here a level's x goes to a ring in the LDS (slot: position in the sweep's
+// order modulo kRing), so a level waits for LDS traffic only, and everything
+// that does not depend on x is loaded one level ahead and stays in flight
+// across the barrier.  Four lanes per node, lane c < 3 for scalar row c: a
+// node's kAhead first lower blocks are three values each in registers.  Per
+// level the blocks are stored [block][node], so a load is consecutive over
+// the lanes.  A scalar row's products are subtracted in the same order as by
+// one thread per node.
+//   lvl       per level: first position, nodes, first padded block, blocks per
+//             node (the most any node of the level has)
+//   lo_ring   per padded block, [node][block]: 3 times the ring slot of its
+//             column (kAhead are read from a node's first on)
+//   lo_val    9 values per padded block
+//   lo_cnt    per position: the node's lower blocks
+//   dinv, rhs per position; node: the internal node at a position
+// Used where every column a level reads is among the kRing positions up to
+// the level's end (the caller checks); a level past 256 nodes runs in passes.
+// Measured on a beam of 3,402 nodes in 148 levels: an iteration 443 -> 222 us
+// (with the wait merged below); what is left per level is the load path of
+// one CU, about 35 bytes a cycle.
+constexpr int kRing = 6400;  // 150 KB of x; the 44,541-node beam's levels read at most 881 positions back
+constexpr int kAhead = 9;    // a node of the beams has at most 9 lower blocks
+constexpr int kRingThreads = 512;
+struct SweepLevel {
+  int t0, count, base, blocks;
+};
+struct SweepItem {
+  int t, cnt, node;
+  bool on;
+  double rhs, d[3], v[kAhead][3];
+  int sl[kAhead];
+};
+__global__ void __launch_bounds__(kRingThreads) ica_sweep_ring(const double *__restrict__ lo_val,
+                                                               const int *__restrict__ lo_ring,
+                                                               const int *__restrict__ lo_cnt,
+                                                               const double *__restrict__ dinv,
+                                                               const double *__restrict__ rhs,
+                                                               const int *__restrict__ node, double *x,
+                                                               const SweepLevel *__restrict__ lvl, int n_levels) {
+  extern __shared__ double ring[];
+  const int kNodes = (int)blockDim.x / 4;
+  const int q0 = (int)threadIdx.x / 4, c = min((int)threadIdx.x % 4, 2);
+  // Every lane issues every load (past the level's nodes or a node's blocks:
+  // its last ones again): with loads under a branch the number in flight is
+  // not known where their values are used, and the wait there would be for
+  // the next item's loads too.
+  auto load = [&](SweepItem &it, const SweepLevel &L, int pass) {
+    const int q = min(pass * kNodes + q0, L.count - 1);
+    it.on = pass * kNodes + q0 < L.count;
+    it.t = L.t0 + q;
+    it.cnt = lo_cnt[it.t];
+    it.node = node[it.t];
+    it.rhs = rhs[3 * (size_t)it.t + c];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) it.d[e] = dinv[9 * (size_t)it.t + 3 * c + e];
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b) {
+      it.sl[b] = lo_ring[(size_t)L.base + (size_t)q * L.blocks + b];
+      const double *v = lo_val + 9 * ((size_t)L.base + (size_t)max(min(b, L.blocks - 1), 0) * L.count + q) + 3 * c;
+#pragma unroll
+      for (int e = 0; e < 3; ++e) it.v[b][e] = v[e];
+    }
+  };
+  auto run = [&](const SweepItem &it, const SweepLevel &L, int pass) {
+    double r = it.rhs;
+    double xb[kAhead][3];
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b)
+#pragma unroll
+      for (int e = 0; e < 3; ++e) xb[b][e] = ring[it.sl[b] + e];
+#pragma unroll
+    for (int b = 0; b < kAhead; ++b) {
+      if (b < it.cnt) {
+        r -= it.v[b][0] * xb[b][0];
+        r -= it.v[b][1] * xb[b][1];
+        r -= it.v[b][2] * xb[b][2];
+      }
+    }
+    for (int b = kAhead; b < it.cnt; ++b) {
+      const int q = min(pass * kNodes + q0, L.count - 1);
+      const double *xe = ring + lo_ring[(size_t)L.base + (size_t)q * L.blocks + b];
+      const double *v = lo_val + 9 * ((size_t)L.base + (size_t)b * L.count + q) + 3 * c;
+      r -= v[0] * xe[0];
+      r -= v[1] * xe[1];
+      r -= v[2] * xe[2];
+    }
+    const double r0 = quad_lane<0>(r), r1 = quad_lane<1>(r), r2 = quad_lane<2>(r);
+    const double xr = it.d[0] * r0 + it.d[1] * r1 + it.d[2] * r2;
+    if (it.on) {  // the quad's fourth lane stores the third's value
+      ring[3 * (it.t % kRing) + c] = xr;
+      x[3 * (size_t)it.node + c] = xr;
+    }
+  };
+  if (n_levels <= 0) return;
+  SweepLevel ahead = lvl[min(1, n_levels - 1)];
+  // items in order: each level's passes; a barrier ends a level
+  auto next = [&](int &lv, int &pass, SweepLevel &L) {  // false past the end
+    if ((pass + 1) * kNodes < L.count) {
+      ++pass;
+      return true;
+    }
+    if (lv + 1 >= n_levels) return false;
+    pass = 0;
+    ++lv;
+    L = ahead;
+    ahead = lvl[min(lv + 1, n_levels - 1)];  // in time for the next level
+    return true;
+  };
+  auto end_level = [&]() {
+    // the level's LDS writes before the next level's reads; loads and stores
+    // of global memory stay in flight (each x is read back from the LDS)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  SweepItem a, b;
+  int la = 0, pa = 0;
+  SweepLevel La = lvl[0];
+  load(a, La, 0);
+  for (;;) {
+    int lb = la, pb = pa;
+    SweepLevel Lb = La;
+    const bool more_b = next(lb, pb, Lb);
+    load(b, Lb, pb);  // past the end: the last item again, not run
+    run(a, La, pa);
+    if (!more_b) break;
+    if (lb != la) end_level();
+    la = lb;
+    pa = pb;
+    La = Lb;
+    const bool more_a = next(la, pa, La);
+    load(a, La, pa);
+    run(b, Lb, pb);
+    if (!more_a) break;
+    if (la != lb) end_level();
+  }
+}
+
+// The padded blocks' values in the ring sweep's order, gathered once per call
+// from their SELL slots (slot < 0: padding, not read).
+__global__ void __launch_bounds__(256) ica_ring_vals(const double *__restrict__ val, const int *__restrict__ lo_slot,
+                                                     int n_pad, double *__restrict__ lo_val) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n_pad) return;
+  const long long slot = lo_slot[p];
+  if (slot < 0) return;
+  const double *v = val + (9 * slot - 8 * (slot % kSlice));
+#pragma unroll
+  for (int k = 0; k < 9; ++k) lo_val[9 * (size_t)p + k] = v[k * kSlice];
+}
+
+// Da^-1 in the sweep's order.
+__global__ void __launch_bounds__(256) ica_order_dinv(const double *__restrict__ dinv, const int *__restrict__ node,
+                                                      int n_nodes, double *__restrict__ out) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= 9 * n_nodes) return;
+  out[k] = dinv[9 * (size_t)node[k / 9] + k % 9];
+}
 
 // ---------------------------------------------------------------- host side
 
@@ -351,7 +523,8 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
   }
   // each level-ordered node's lower blocks (nodes before it), in block
   // order: SELL slot and column
-  std::vector<int> lo_ptr(nn + 1, 0), lo_slot, lo_col;
+  std::vector<int> lo_ptr(nn + 1, 0), lo_slot, lo_col, pos(nn);
+  for (int t = 0; t < nn; ++t) pos[lvl_node[t]] = t;
   for (int t = 0; t < nn; ++t) {
     const int i = lvl_node[t], u = A->perm[i], sl = i / kSlice, l = i % kSlice;
     const int b0 = A->sl_off_h[sl], W = (A->sl_off_h[sl + 1] - b0) / kSlice;
@@ -364,14 +537,55 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
     }
     lo_ptr[t + 1] = (int)lo_slot.size();
   }
-  const size_t n_lo = lo_slot.size();
+  size_t n_lo = lo_slot.size();
+  // the ring sweep's levels, if every column a level reads is within kRing
+  // positions of the level's end and the padded blocks stay few
+  std::vector<SweepLevel> lvl(n_levels);
+  std::vector<int> lo_cnt(nn), lo_ring;
+  bool use_ring = true;
+  int ring_threads = 64;
+  size_t n_pad = 0;
+  for (int lv = 0; lv < n_levels; ++lv) {
+    int most = 0;
+    for (int t = lvl_ptr[lv]; t < lvl_ptr[lv + 1]; ++t) {
+      lo_cnt[t] = lo_ptr[t + 1] - lo_ptr[t];
+      most = std::max(most, lo_cnt[t]);
+      for (int e = lo_ptr[t]; e < lo_ptr[t + 1]; ++e)
+        use_ring = use_ring && lvl_ptr[lv + 1] - 1 - pos[lo_col[e]] < kRing;
+    }
+    lvl[lv] = SweepLevel{lvl_ptr[lv], lvl_ptr[lv + 1] - lvl_ptr[lv], (int)n_pad, most};
+    n_pad += (size_t)most * lvl[lv].count;
+    use_ring = use_ring && 9 * n_pad < 0x7fffffff;
+  }
+  use_ring = use_ring && n_pad <= 3 * n_lo + 1024;
+  if (use_ring) {
+    // a level without lower blocks reads one block column past its base, a
+    // node's kAhead slots may run past its own
+    int widest = 0;
+    for (const SweepLevel &L : lvl) widest = std::max(widest, L.count);
+    n_pad += widest + kAhead;
+    ring_threads = std::min(kRingThreads, (4 * widest + 63) / 64 * 64);
+    std::vector<int> slot_p(n_pad, -1);
+    lo_ring.assign(n_pad, 0);
+    for (const SweepLevel &L : lvl)
+      for (int qn = 0; qn < L.count; ++qn)
+        for (int b = 0; b < lo_cnt[L.t0 + qn]; ++b) {
+          const size_t e = lo_ptr[L.t0 + qn] + b;
+          slot_p[(size_t)L.base + (size_t)b * L.count + qn] = lo_slot[e];
+          lo_ring[(size_t)L.base + (size_t)qn * L.blocks + b] = 3 * (pos[lo_col[e]] % kRing);
+        }
+    lo_slot.swap(slot_p);
+    lo_col.swap(lo_ring);  // the column list the kernel reads: ring slots
+    n_lo = n_pad;
+  }
 
-  // device block: Da^-1, levels, the lower blocks and their products, J and
+  // device block: Da^-1, levels, the lower blocks and their values, J and
   // J^T, J u, lambda, dot partials
   const size_t parts = ((size_t)n + 255) / 256 + 1;
-  const size_t bytes = sizeof(double) * (9 * (size_t)nn + 9 * n_lo + 2 * (size_t)nnz + 2 * (size_t)m + parts + 8) +
-                       sizeof(int) * ((size_t)n_levels + 1 + (size_t)nn + (size_t)nn + 1 + 2 * n_lo + (size_t)m +
-                                      1 + 2 * (size_t)nnz + (size_t)n + 1) +
+  const size_t bytes = sizeof(double) * ((use_ring ? 18 : 9) * (size_t)nn + 9 * n_lo + 2 * (size_t)nnz + 2 * (size_t)m +
+                                         parts + 8) +
+                       sizeof(int) * ((size_t)n_levels + 1 + 3 * ((size_t)nn + 1) + 2 * n_lo + 4 * (size_t)n_levels +
+                                      (size_t)m + 1 + 2 * (size_t)nnz + (size_t)n + 1) +
                        1024;
   void *blk = nullptr;
   if (int rc = ctx->alloc(&blk, bytes)) return rc;
@@ -396,13 +610,15 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
   double *d_jx = (double *)carve(sizeof(double) * (m + 1));
   double *d_lam = (double *)carve(sizeof(double) * (m + 1));
   double *d_part = (double *)carve(sizeof(double) * parts);
-  double *d_res = (double *)carve(sizeof(double) * 8);
   int *d_lvl_ptr = (int *)carve(sizeof(int) * (n_levels + 1));
   int *d_lvl_node = (int *)carve(sizeof(int) * (size_t)nn);
   double *d_lo_val = (double *)carve(sizeof(double) * 9 * n_lo);
   int *d_lo_ptr = (int *)carve(sizeof(int) * ((size_t)nn + 1));
   int *d_lo_slot = (int *)carve(sizeof(int) * n_lo);
   int *d_lo_col = (int *)carve(sizeof(int) * n_lo);
+  double *d_dinv_t = use_ring ? (double *)carve(sizeof(double) * 9 * (size_t)nn) : nullptr;
+  SweepLevel *d_lvl = (SweepLevel *)carve(sizeof(SweepLevel) * (size_t)n_levels);
+  int *d_pos = (int *)carve(sizeof(int) * (size_t)nn);
   int *d_jp = (int *)carve(sizeof(int) * (m + 1));
   int *d_jc = (int *)carve(sizeof(int) * nnz);
   int *d_tp = (int *)carve(sizeof(int) * (n + 1));
@@ -417,7 +633,15 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
   MPRGP_HIP(hipMemcpyAsync(d_tp, Ri.tptr.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, s));
   MPRGP_HIP(hipMemcpyAsync(d_lvl_ptr, lvl_ptr.data(), sizeof(int) * (n_levels + 1), hipMemcpyHostToDevice, s));
   MPRGP_HIP(hipMemcpyAsync(d_lvl_node, lvl_node.data(), sizeof(int) * (size_t)nn, hipMemcpyHostToDevice, s));
-  MPRGP_HIP(hipMemcpyAsync(d_lo_ptr, lo_ptr.data(), sizeof(int) * ((size_t)nn + 1), hipMemcpyHostToDevice, s));
+  if (use_ring) {
+    MPRGP_HIP(hipMemcpyAsync(d_lo_ptr, lo_cnt.data(), sizeof(int) * (size_t)nn, hipMemcpyHostToDevice, s));
+    MPRGP_HIP(hipMemcpyAsync(d_lvl, lvl.data(), sizeof(SweepLevel) * (size_t)n_levels, hipMemcpyHostToDevice, s));
+    MPRGP_HIP(hipMemcpyAsync(d_pos, pos.data(), sizeof(int) * (size_t)nn, hipMemcpyHostToDevice, s));
+    MPRGP_HIP(hipFuncSetAttribute((const void *)ica_sweep_ring, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  3 * kRing * (int)sizeof(double)));
+  } else {
+    MPRGP_HIP(hipMemcpyAsync(d_lo_ptr, lo_ptr.data(), sizeof(int) * ((size_t)nn + 1), hipMemcpyHostToDevice, s));
+  }
   if (n_lo > 0) {
     MPRGP_HIP(hipMemcpyAsync(d_lo_slot, lo_slot.data(), sizeof(int) * n_lo, hipMemcpyHostToDevice, s));
     MPRGP_HIP(hipMemcpyAsync(d_lo_col, lo_col.data(), sizeof(int) * n_lo, hipMemcpyHostToDevice, s));
@@ -427,14 +651,21 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
     ica_dinv<<<blocks, 256, 0, s>>>(A->d_sl_off, A->d_col, A->d_val, nn, d_dinv);
     MPRGP_HIP(hipGetLastError());
   }
-  if (n_lo > 0) {
+  if (use_ring && nn > 0) {
+    ica_order_dinv<<<(9 * nn + 255) / 256, 256, 0, s>>>(d_dinv, d_lvl_node, nn, d_dinv_t);
+    MPRGP_HIP(hipGetLastError());
+  }
+  if (n_lo > 0 && use_ring) {
+    ica_ring_vals<<<(unsigned)((n_lo + 255) / 256), 256, 0, s>>>(A->d_val, d_lo_slot, (int)n_lo, d_lo_val);
+    MPRGP_HIP(hipGetLastError());
+  } else if (n_lo > 0) {
     ica_lower_vals<<<(unsigned)((n_lo + 255) / 256), 256, 0, s>>>(A->d_val, d_lo_slot, (int)n_lo, d_lo_val);
     MPRGP_HIP(hipGetLastError());
   }
   // B = J Da^-1 J^T on the host, from the inverse blocks in user order
   std::vector<RowNodes> rows;
   HostCsr B;
-  std::vector<double> invd(m, 0.0), c(m), lam(m, 0.0), rhs(m), pre(m), jx(m);
+  std::vector<double> invd(m, 0.0), c(m), lam(m, 0.0), rhs(m), pre(m);
   if (m > 0) {
     std::vector<double> dinv((size_t)9 * nn), dinv_user((size_t)9 * nn);
     MPRGP_HIP(hipMemcpyAsync(dinv.data(), d_dinv, sizeof(double) * dinv.size(), hipMemcpyDeviceToHost, s));
@@ -449,41 +680,73 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
   }
   double *u = q->z, *jtl = q->phi, *rh = q->beta, *e = q->ap;
   const double *x_c = q->x;
+  // pinned: J u and the residual as read back (d_jx, m + 1 doubles), lambda
+  struct Pinned {
+    double *p = nullptr;
+    ~Pinned() {
+      if (p) (void)hipHostFree(p);
+    }
+  } pin;
+  if (hipHostMalloc((void **)&pin.p, sizeof(double) * (2 * (size_t)m + 1), hipHostMallocDefault) != hipSuccess) {
+    pin.p = nullptr;
+    (void)hipGetLastError();
+    return fail(MPRGP_ENOMEM, "pinned staging of %d multipliers", m);
+  }
+  double *h_jx = pin.p, *h_lam = pin.p + m + 1, *d_r2 = d_jx + m;
+  Release drain_{ctx, nullptr, 0};  // before the pinned block goes: an upload from it may be queued
   MPRGP_HIP(hipMemsetAsync(jtl, 0, sizeof(double) * n, s));
-  MPRGP_HIP(hipMemsetAsync(d_res, 0, sizeof(double) * 8, s));
+  MPRGP_HIP(hipMemsetAsync(d_jx, 0, sizeof(double) * ((size_t)m + 1), s));
   MPRGP_HIP(hipEventRecord(ctx->t0, s));
   int it = 0, sweeps = 0;
   bool met = false;
   double residual = -1.0;
+  // J u for the next c = p + J Da^-1 (LaUa x - b), queued behind the sweep
+  // that makes its x, so that one wait per iteration brings it back with the
+  // residual (after the last sweep it is not used)
+  auto queue_ju = [&]() -> int {
+    ica_rows<<<blocks, 256, 0, s>>>(A->d_sl_off, A->d_col, A->d_val, A->d_perm, x_c, q->b, jtl, d_dinv, u, nn,
+                                    kOffDiag, nullptr);
+    MPRGP_HIP(hipGetLastError());
+    MPRGP_HIP(launch_csr_mul(s, m, d_jp, d_jc, d_jv, u, d_jx));
+    return MPRGP_OK;
+  };
+  auto read_back = [&]() -> int {
+    MPRGP_HIP(hipMemcpyAsync(h_jx, d_jx, sizeof(double) * ((size_t)m + 1), hipMemcpyDeviceToHost, s));
+    MPRGP_HIP(hipStreamSynchronize(s));
+    return MPRGP_OK;
+  };
+  if (m > 0 && max_it > 0) {
+    if (int rc = queue_ju()) return rc;
+    if (int rc = read_back()) return rc;
+  }
   for (it = 0; it < max_it; ++it) {
     if (m > 0) {
-      ica_rows<<<blocks, 256, 0, s>>>(A->d_sl_off, A->d_col, A->d_val, A->d_perm, x_c, q->b, jtl, d_dinv, u, nn,
-                                      kOffDiag);
-      MPRGP_HIP(hipGetLastError());
-      MPRGP_HIP(launch_csr_mul(s, m, d_jp, d_jc, d_jv, u, d_jx));
-      MPRGP_HIP(hipMemcpyAsync(jx.data(), d_jx, sizeof(double) * m, hipMemcpyDeviceToHost, s));
-      MPRGP_HIP(hipStreamSynchronize(s));
-      for (int i = 0; i < m; ++i) c[i] = p[i] + jx[i];
+      for (int i = 0; i < m; ++i) c[i] = p[i] + h_jx[i];
       sweeps += pgs(B, invd, c, lam, gs_max_it, gs_tol, rhs, pre);
-      MPRGP_HIP(hipMemcpyAsync(d_lam, lam.data(), sizeof(double) * m, hipMemcpyHostToDevice, s));
+      std::copy(lam.begin(), lam.end(), h_lam);
+      MPRGP_HIP(hipMemcpyAsync(d_lam, h_lam, sizeof(double) * m, hipMemcpyHostToDevice, s));
       MPRGP_HIP(launch_csr_mul(s, n, d_tp, d_tc, d_tv, d_lam, jtl));
     }
     if (nn > 0) {
       ica_rows<<<blocks, 256, 0, s>>>(A->d_sl_off, A->d_col, A->d_val, A->d_perm, x_c, q->b, jtl, d_dinv, rh, nn,
-                                      kUpper);
+                                      kUpper, use_ring ? d_pos : nullptr);
       MPRGP_HIP(hipGetLastError());
-      ica_sweep<<<1, kSweepThreads, 0, s>>>(d_lo_val, d_lo_col, d_lo_ptr, d_dinv, rh, q->x, d_lvl_ptr,
-                                            d_lvl_node, n_levels);
+      if (use_ring)
+        ica_sweep_ring<<<1, ring_threads, 3 * kRing * sizeof(double), s>>>(d_lo_val, d_lo_col, d_lo_ptr, d_dinv_t, rh,
+                                                                           d_lvl_node, q->x, d_lvl, n_levels);
+      else
+        ica_sweep<<<1, kSweepThreads, 0, s>>>(d_lo_val, d_lo_col, d_lo_ptr, d_dinv, rh, q->x, d_lvl_ptr,
+                                              d_lvl_node, n_levels);
       MPRGP_HIP(hipGetLastError());
       ica_rows<<<blocks, 256, 0, s>>>(A->d_sl_off, A->d_col, A->d_val, A->d_perm, x_c, q->b, jtl, d_dinv, e, nn,
-                                      kResidual);
+                                      kResidual, nullptr);
       MPRGP_HIP(hipGetLastError());
     }
-    MPRGP_HIP(launch_dot(s, e, e, (size_t)n, d_part, d_res));
-    double r2 = 0.0;
-    MPRGP_HIP(hipMemcpyAsync(&r2, d_res, sizeof(double), hipMemcpyDeviceToHost, s));
-    MPRGP_HIP(hipStreamSynchronize(s));  // also completes the lambda upload before the next PGS
-    residual = std::sqrt(r2);
+    MPRGP_HIP(launch_dot(s, e, e, (size_t)n, d_part, d_r2));
+    if (m > 0 && it + 1 < max_it)
+      if (int rc = queue_ju()) return rc;
+    if (int rc = read_back()) return rc;
+    residual = std::sqrt(h_jx[m]);
     if (residual <= tol) {
       met = true;
       break;
