@@ -16,7 +16,10 @@
 // once per solve.  Each of these decisions reads a few device scalars or an
 // m-vector back, so a solve synchronises the stream a few times per
 // iteration: this path is for coupled rows, which the simulator's decoupled
-// solve (the batched kernels) does not have.
+// solve (the batched kernels) does not have.  Where the rows' components are
+// small and the system fits one CU (mprgp_general.h), the main loop runs in
+// one workgroup instead (mprgp_general_dev.hip), and the host drives only the
+// start, the power method and the final projection.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,6 +27,7 @@
 #include <cstring>
 #include <vector>
 
+#include "mprgp_general.h"
 #include "mprgp_host.h"
 
 using namespace mprgp;
@@ -265,6 +269,64 @@ struct General {
     }
     if (!qp_nonneg(k, Gk, hk, lk, tol)) qp_fail = true;
     for (int a = 0; a < k; ++a) l[rows[a]] = lk.empty() ? 0.0 : lk[a];
+  }
+
+  // The one-workgroup loop (mprgp_general_dev.hip) takes the main loop: its
+  // components, packed, and its share of the device block.
+  bool one_launch = false;
+  std::vector<int> big_row, one_row;
+  std::vector<double> big_g, one_g;
+  GenArgs *d_args = nullptr;
+  GenState *d_state = nullptr;
+  double *d_c = nullptr, *d_big_g = nullptr, *d_one_g = nullptr;
+  int *d_big_row = nullptr, *d_one_row = nullptr;
+  unsigned char *d_face = nullptr;
+  void pack_components(int n_nodes) {
+    one_launch = m > 0 && m <= kGenMaxRows && n_nodes <= kGenMaxNodes;
+    for (const auto &rows : comps) one_launch = one_launch && rows.size() <= (size_t)kGenBlock;
+    if (!one_launch) return;
+    for (size_t c0 = 0; c0 < comps.size(); ++c0) {
+      const int k = (int)comps[c0].size();
+      if (k == 1) {
+        one_row.push_back(comps[c0][0]);
+        one_g.push_back(gc[c0][0]);
+        continue;
+      }
+      for (int i = 0; i < kGenBlock; ++i) {
+        big_row.push_back(i < k ? comps[c0][i] : -1);
+        for (int j = 0; j < kGenBlock; ++j) big_g.push_back(i < k && j < k ? gc[c0][(size_t)i * k + j] : 0.0);
+      }
+    }
+  }
+  // The main loop from the current g, phi, z, p and face, kGenChunk
+  // iterations a launch; st: its counters.
+  int loop_on_device(double alpha_bar, double tol, int max_it, bool pre, GenState *st) {
+    const mprgp_matrix *A = q->A;
+    const GenArgs a{n, m, A->n_nodes, A->n_slices, A->d_sl_off, A->d_col, A->d_val, dinv, b, x, g, p, z, phi, beta,
+                    y, gp, t, t2, t3, tl, jp, jc, tp, tc, jv, tv, d_c, d_face, jslot(0), jslot(1), lam, lam + m + 1, part,
+                    (int)big_row.size() / kGenBlock, (int)one_row.size(), d_big_row, d_one_row, d_big_g, d_one_g,
+                    alpha_bar, tol, max_it, pre, kGenChunk, d_state};
+    *st = GenState{};
+    MPRGP_HIP(hipMemcpyAsync(d_args, &a, sizeof(a), hipMemcpyHostToDevice, s));
+    MPRGP_HIP(hipMemcpyAsync(d_state, st, sizeof(*st), hipMemcpyHostToDevice, s));
+    MPRGP_HIP(hipMemcpyAsync(d_face, face.data(), (size_t)m, hipMemcpyHostToDevice, s));
+    MPRGP_HIP(hipStreamSynchronize(s));  // a is a local
+    while (!st->done && !st->fail) {
+      MPRGP_HIP(launch_general_loop(s, d_args));
+      MPRGP_HIP(hipMemcpyAsync(h_rb, d_state, sizeof(*st), hipMemcpyDeviceToHost, s));
+      MPRGP_HIP(hipStreamSynchronize(s));
+      std::memcpy(st, h_rb, sizeof(*st));
+    }
+    MPRGP_HIP(hipMemcpyAsync(h_rb, d_face, (size_t)m, hipMemcpyDeviceToHost, s));
+    MPRGP_HIP(hipStreamSynchronize(s));
+    std::memcpy(face.data(), h_rb, (size_t)m);
+    act.clear();
+    for (int i = 0; i < m; ++i)
+      if (face[i]) act.push_back(i);
+    if (st->fail) qp_fail = true;
+    y_size = st->y_set ? n : 0;
+    jx_ok = jy_ok = false;
+    return MPRGP_OK;
   }
 
   // Pinned host memory: the multipliers' staging (two slots of m + 1) and
@@ -624,10 +686,14 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
   G.c.assign(c, c + m);
   if (int rc = G.build_jjt(j_ptr, j_val, jc, tptr, tc)) return rc;
   G.face.assign(m, 0);
+  G.pack_components(q->n);
   // device block: J, J^T, J v, lambda, dot partials and results
   const size_t parts = ((size_t)n + 255) / 256 + 1;
   const size_t bytes = sizeof(int) * ((size_t)m + 1 + (size_t)nnz + (size_t)n + 1 + (size_t)nnz) +
-                       sizeof(double) * (2 * (size_t)nnz + 5 * ((size_t)m + 1) + kMaxDots * parts + 16) + 1024;
+                       sizeof(double) * (2 * (size_t)nnz + 5 * ((size_t)m + 1) + kMaxDots * parts + 16) + 1024 +
+                       (G.one_launch ? sizeof(GenArgs) + sizeof(GenState) + sizeof(double) * (G.big_g.size() + 2 * (size_t)m) +
+                                           sizeof(int) * (G.big_row.size() + (size_t)m) + (size_t)m
+                                     : 0);
   if (int rc = ctx->alloc(&G.blk, bytes)) return rc;
   G.blk_bytes = bytes;
   if (hipHostMalloc((void **)&G.h_lam, sizeof(double) * (5 * ((size_t)m + 1) + 16), hipHostMallocDefault) !=
@@ -653,6 +719,16 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
     G.jc = (int *)carve(sizeof(int) * nnz);
     G.tp = (int *)carve(sizeof(int) * (n + 1));
     G.tc = (int *)carve(sizeof(int) * nnz);
+    if (G.one_launch) {
+      G.d_args = (GenArgs *)carve(sizeof(GenArgs));
+      G.d_state = (GenState *)carve(sizeof(GenState));
+      G.d_c = (double *)carve(sizeof(double) * m);
+      G.d_big_g = (double *)carve(sizeof(double) * G.big_g.size());
+      G.d_one_g = (double *)carve(sizeof(double) * G.one_g.size());
+      G.d_big_row = (int *)carve(sizeof(int) * G.big_row.size());
+      G.d_one_row = (int *)carve(sizeof(int) * G.one_row.size());
+      G.d_face = (unsigned char *)carve(m);
+    }
   }
   hipStream_t s = G.s;
   if (m > 0) {
@@ -663,6 +739,17 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
     MPRGP_HIP(hipMemcpyAsync(G.tv, tv.data(), sizeof(double) * nnz, hipMemcpyHostToDevice, s));
   }
   MPRGP_HIP(hipMemcpyAsync(G.tp, tptr.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, s));
+  if (G.one_launch) {
+    MPRGP_HIP(hipMemcpyAsync(G.d_c, c, sizeof(double) * m, hipMemcpyHostToDevice, s));
+    if (!G.big_row.empty()) {
+      MPRGP_HIP(hipMemcpyAsync(G.d_big_g, G.big_g.data(), sizeof(double) * G.big_g.size(), hipMemcpyHostToDevice, s));
+      MPRGP_HIP(hipMemcpyAsync(G.d_big_row, G.big_row.data(), sizeof(int) * G.big_row.size(), hipMemcpyHostToDevice, s));
+    }
+    if (!G.one_row.empty()) {
+      MPRGP_HIP(hipMemcpyAsync(G.d_one_g, G.one_g.data(), sizeof(double) * G.one_g.size(), hipMemcpyHostToDevice, s));
+      MPRGP_HIP(hipMemcpyAsync(G.d_one_row, G.one_row.data(), sizeof(int) * G.one_row.size(), hipMemcpyHostToDevice, s));
+    }
+  }
   MPRGP_HIP(hipStreamSynchronize(s));  // the host arrays above are locals
   G.x = q->x; G.g = q->g; G.p = q->p; G.z = q->z; G.phi = q->phi; G.beta = q->beta; G.y = q->y;
   G.gp = q->ap; G.t = q->py; G.t2 = q->p2; G.t3 = q->beta2; G.tl = q->pu; G.pv = q->pv; G.pw = q->pw;
@@ -735,7 +822,16 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
   if (int rc = G.precond(pre)) return rc;
   MPRGP_HIP(hipMemcpyAsync(G.p, G.z, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   double *AP = G.gp;  // A p shares gp's buffer: gp is read only by its own sum
-  for (iteration = 0; iteration < p.max_it;) {
+  if (G.one_launch) {
+    GenState st;
+    if (int rc = G.loop_on_device(alpha_bar, tol, p.max_it, pre, &st)) return rc;
+    residual = st.residual;
+    iteration = st.iteration;
+    num_cg = st.num_cg;
+    num_exp = st.num_exp;
+    num_prop = st.num_prop;
+  }
+  for (; !G.one_launch && iteration < p.max_it;) {
     // computeGradients (:163-173) with phi current, then proportional at x
     if (int rc = G.head_launch(G.x, alpha_bar, m > 0 && G.y_size > 0)) return rc;
     if (int rc = G.head_wait(0)) return rc;

@@ -1,0 +1,48 @@
+// mprgp_general.h -- the one-workgroup main loop of the coupled-row solve
+// (mprgp_general_dev.hip), as mprgp_general.cpp drives it.
+#pragma once
+#include "mprgp_host.h"
+
+namespace mprgp {
+
+// Rows of the largest component (rows that share nodes) the one-workgroup loop
+// takes: a vertex-triangle contact row and the plane rows of its four nodes
+// are five.  A component's QP runs in one thread's registers.
+constexpr int kGenBlock = 6;
+// Nodes of the largest system: the vector a product gathers from is 24 bytes
+// a node of the 64 KB a kernel declares.  There the loop is still the faster
+// one, 271 ms against 570 ms from the host over 1,001 iterations at 2,499
+// nodes, but its products with A, on one CU, grow with the matrix.
+constexpr int kGenMaxNodes = 2600;
+constexpr int kGenMaxRows = 16384;  // some two rows per entry of the largest vector
+// Iterations per launch, so that no launch runs long.
+constexpr int kGenChunk = 256;
+
+struct GenState {
+  int in_cg;  // the launch ended between two steps of the CG loop, else at the outer loop's head
+  int iteration, num_cg, num_exp, num_prop;
+  int prop, y_set, ax_set, done, fail;
+  double residual, alpha, fx, fy;
+};
+
+struct GenArgs {
+  int n, m, n_nodes, n_slices;
+  const int *sl_off, *col;
+  const double *val, *dinv, *b;
+  double *x, *g, *p, *z, *phi, *beta, *y, *ap, *t, *t2, *t3, *ax;
+  const int *jp, *jc, *tp, *tc;
+  const double *jv, *tv, *c;
+  unsigned char *face;                  // per row, as the last face decision left it
+  double *j1, *j2, *lam, *lam2, *part;  // m, m, m, m; 8 per 256 entries
+  // components of several rows: row numbers (-1: none) and J J^T, padded to
+  // kGenBlock; components of one row
+  int n_big, n_one;
+  const int *big_row, *one_row;
+  const double *big_g, *one_g;
+  double alpha_bar, tol;
+  int max_it, pre, chunk;
+  GenState *st;
+};
+hipError_t launch_general_loop(hipStream_t s, const GenArgs *args);  // args in device memory
+
+}  // namespace mprgp
