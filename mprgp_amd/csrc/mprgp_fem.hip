@@ -5,13 +5,12 @@
 //
 // Three passes, no atomics, every sum in tet order so the result is
 // deterministic and independent of the launch shape:
-//   1. fem_element: one thread per tet computes h^2 K_e (16 blocks of 3x3)
-//      and h^2 f_e (4 x 3) into a scratch array laid out [entry][tet] so the
-//      per-thread writes are coalesced.
-//   2. fem_blocks: one thread per block of A sums the contributions of the
-//      tets sharing that node pair (a precomputed list in tet order), adds
-//      the lumped mass on diagonal blocks and stores the block straight into
-//      its SELL-64 slot.
+//   1. fem_element: one thread per tet computes h^2 f_e (4 x 3) and the 31
+//      numbers that the 16 blocks of K_e are made of.
+//   2. fem_blocks: one thread per block of A forms and sums the contributions
+//      of the tets sharing that node pair (a precomputed list in tet order),
+//      adds the lumped mass on diagonal blocks and stores the block straight
+//      into its SELL-64 slot.
 //   3. fem_rhs: one thread per node sums its tets' forces, gravity and the
 //      inertia term; A x_n is then added by the SELL SpMV.
 //
@@ -29,6 +28,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -39,10 +39,30 @@
 
 namespace mprgp {
 
-// per tet, contiguous (tet-major, so a block's 9 values are one read for the
-// kernels that sum them): kc K_e blocks, then h^2 f_e, then K_e c_e (the
-// damping term)
-constexpr int kElemOut = 16 * 9 + 12 + 12;
+// Per tet, contiguous.  K_e's record, 256 bytes: u_I (12), R R^T's lower
+// triangle (6), V, lambda, mu, and B_I.B_J's lower triangle (10); the forces
+// h^2 f_e (12) and K_e c_e (the damping term, 12) of all tets follow.  The 16
+// blocks themselves are 144 numbers, 230 MB for 200,000 tets against the
+// records' 51 MB: written by fem_element, read by fem_blocks, they took the
+// two 172 and 132 us, the records 72 and 72 us.  A block is 70 operations,
+// formed by the thread that sums it.
+constexpr int kRec = 32, kRecRR = 12, kRecV = 18, kRecBB = 21;
+constexpr int kElemOut = kRec + 12 + 12;
+__host__ __device__ constexpr int low(int i, int j) { return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; }
+
+// The workgroup's share of the work: consecutive workgroups run on different
+// XCDs, so each XCD is given a run of neighbouring shares, whose tets its L2
+// then holds once.
+__device__ __forceinline__ int near_block() {
+  const int x = blockIdx.x % 8, per = gridDim.x / 8, more = gridDim.x % 8;
+  return x * per + min(x, more) + blockIdx.x / 8;
+}
+
+// Entry (r, s) of V [ lambda u_I u_J^T + mu ((R R^T)(B_I.B_J) + u_J u_I^T) ].
+__device__ __forceinline__ double stiffness(double V, double lam, double mu, const double *uI, const double *uJ,
+                                            double rr, double bb, int r, int s) {
+  return V * (lam * uI[r] * uJ[s] + mu * (rr * bb + uJ[r] * uI[s]));
+}
 
 __device__ inline double det3(const double *M) {
   return M[0] * (M[4] * M[8] - M[5] * M[7]) - M[1] * (M[3] * M[8] - M[5] * M[6]) +
@@ -248,51 +268,101 @@ __global__ void __launch_bounds__(128) fem_element(int T, const int4 *__restrict
       for (int c = 0; c < 3; ++c) s += R[r * 3 + c] * B[I][c];
       u[I][r] = s;
     }
-  // kc K_e blocks; K_e c_e for the damping term
-  double ce[12];
-  if (damp)
+  double *rec = out + (size_t)t * kRec, *force = out + (size_t)T * kRec + (size_t)t * 12;
+  double *dampf = out + (size_t)T * (kRec + 12) + (size_t)t * 12;
+  double bb[10];
+  for (int I = 0; I < 4; ++I)
+    for (int J = 0; J <= I; ++J) bb[low(I, J)] = (B[I][0] * B[J][0] + B[I][1] * B[J][1]) + B[I][2] * B[J][2];
+  if (!rhs_only) {
+    for (int I = 0; I < 4; ++I)
+      for (int r = 0; r < 3; ++r) rec[I * 3 + r] = u[I][r];
+    for (int r = 0; r < 3; ++r)
+      for (int c = 0; c <= r; ++c) rec[kRecRR + low(r, c)] = RRt[r * 3 + c];
+    rec[kRecV] = V;
+    rec[kRecV + 1] = lam;
+    rec[kRecV + 2] = mu;
+    for (int e = 0; e < 10; ++e) rec[kRecBB + e] = bb[e];
+  }
+  if (damp) {  // K_e c_e
+    double ce[12];
     for (int i = 0; i < 4; ++i)
       for (int r = 0; r < 3; ++r) ce[i * 3 + r] = (xn[3 * (size_t)vi[i] + r] - xe[i * 3 + r]) * h;
-  for (int I = 0; I < 4 && (!rhs_only || damp); ++I) {
-    double kd[3] = {0.0, 0.0, 0.0};
-    for (int J = 0; J < 4; ++J) {
-      const double bb = (B[I][0] * B[J][0] + B[I][1] * B[J][1]) + B[I][2] * B[J][2];
-      for (int r = 0; r < 3; ++r)
-        for (int s = 0; s < 3; ++s) {
-          double k = V * (lam * u[I][r] * u[J][s] + mu * (RRt[r * 3 + s] * bb + u[J][r] * u[I][s]));
-          if (!rhs_only) out[(size_t)t * kElemOut + ((I * 4 + J) * 9) + r * 3 + s] = k * kc;
-          if (damp) kd[r] += k * ce[J * 3 + s];
-        }
+    for (int I = 0; I < 4; ++I) {
+      double kd[3] = {0.0, 0.0, 0.0};
+      for (int J = 0; J < 4; ++J)
+        for (int r = 0; r < 3; ++r)
+          for (int s = 0; s < 3; ++s)
+            kd[r] += stiffness(V, lam, mu, u[I], u[J], RRt[r * 3 + s], bb[low(I, J)], r, s) * ce[J * 3 + s];
+      for (int r = 0; r < 3; ++r) dampf[I * 3 + r] = kd[r];
     }
-    if (damp)
-      for (int r = 0; r < 3; ++r) out[(size_t)t * kElemOut + 156 + I * 3 + r] = kd[r];
   }
   // h^2 f_e
   for (int I = 0; I < 4; ++I)
     for (int r = 0; r < 3; ++r) {
       double s = 0.0;
       for (int c = 0; c < 3; ++c) s += RP[r * 3 + c] * B[I][c];
-      out[(size_t)t * kElemOut + 144 + I * 3 + r] = -(V * s) * h2;
+      force[I * 3 + r] = -(V * s) * h2;
     }
 }
 
-// One thread per block of A (node-order block index b): sums the tets'
-// h^2 K_e blocks in tet order, adds M on the diagonal, stores the block in
+// One thread per block of A: sums the tets' kc K_e blocks, formed from the
+// tets' records, in tet order, adds M on the diagonal, stores the block in
 // its SELL slot (value base vbase[b], entry planes 64 apart).
-__global__ void fem_blocks(long long nb, int T, const int *__restrict__ ptr, const int *__restrict__ ctr,
-                           const int *__restrict__ vbase, const int *__restrict__ diag_node,
-                           const double *__restrict__ mass, double mc, const double *__restrict__ elem,
-                           double *__restrict__ val) {
-  const long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nb) return;
+//
+// A workgroup's kGroup blocks are those of neighbouring rows, which share
+// their tets: each record is copied to LDS once (a thread reading the records
+// of its own tets makes a cache access for each of 11 loads, 35M accesses for
+// 200,000 tets and 133 us, in this order of the blocks or in that of their
+// slots; 72 us so).  tets: each workgroup's tets, ascending; a
+// contribution names its tet by the place in that list.  Longer lists than
+// LDS holds are taken in runs, which keep the order of the sums.  The
+// workgroup's blocks stand by descending list length, so that the diagonal's
+// (24 tets in a Kuhn mesh, 4 to 6 elsewhere) share a wavefront.
+constexpr int kGroup = 256;  // blocks of A, threads
+constexpr int kHeld = 96;    // records in LDS, 264 bytes apart (40 to 112: 72-78 us; 224, two workgroups a CU: 117 us)
+__global__ void __launch_bounds__(kGroup) fem_blocks(long long nb, const int *__restrict__ ptr, const int *__restrict__ ctr,
+                                                     const int *__restrict__ grp_ptr, const int *__restrict__ grp_tet,
+                                                     const int *__restrict__ vbase, const int *__restrict__ diag_node,
+                                                     const double *__restrict__ mass, double mc, double kc,
+                                                     const double *__restrict__ elem, double *__restrict__ val) {
+  __shared__ double held[kHeld * (kRec + 1)];
+  const int grp = near_block(), tid = threadIdx.x;
+  const long long b = (long long)grp * kGroup + tid;
+  const int t0 = grp_ptr[grp], nt = grp_ptr[grp + 1] - t0;
+  int k = 0, end = 0;
+  if (b < nb) {
+    k = ptr[b];
+    end = ptr[b + 1];
+  }
+  int code = k < end ? ctr[k] : INT_MAX;
   double acc[9];
   for (int e = 0; e < 9; ++e) acc[e] = 0.0;
-  for (int k = ptr[b]; k < ptr[b + 1]; ++k) {
-    const int code = ctr[k];
-    const int t = code >> 4, IJ = code & 15;
-    const double *eb = elem + (size_t)t * kElemOut + IJ * 9;  // the block's 9 values, contiguous
-    for (int e = 0; e < 9; ++e) acc[e] += eb[e];
+  for (int base = 0; base < nt; base += kHeld) {
+    const int here = min(kHeld, nt - base);
+    __syncthreads();
+    for (int i = tid; i < here * (kRec / 2); i += kGroup) {
+      const int r = i / (kRec / 2), e = 2 * (i % (kRec / 2));
+      const double2 v = *(const double2 *)(elem + (size_t)grp_tet[t0 + base + r] * kRec + e);
+      held[r * (kRec + 1) + e] = v.x;
+      held[r * (kRec + 1) + e + 1] = v.y;
+    }
+    __syncthreads();
+    while (code >> 4 < base + here) {
+      const double *q = held + ((code >> 4) - base) * (kRec + 1);
+      const int I = code >> 2 & 3, J = code & 3;
+      code = ++k < end ? ctr[k] : INT_MAX;
+      double uI[3], uJ[3], rr[6];
+      for (int e = 0; e < 3; ++e) {
+        uI[e] = q[3 * I + e];
+        uJ[e] = q[3 * J + e];
+      }
+      for (int e = 0; e < 6; ++e) rr[e] = q[kRecRR + e];
+      const double V = q[kRecV], lam = q[kRecV + 1], mu = q[kRecV + 2], bb = q[kRecBB + low(I, J)];
+      for (int r = 0; r < 3; ++r)
+        for (int c = 0; c < 3; ++c) acc[r * 3 + c] += stiffness(V, lam, mu, uI, uJ, rr[low(r, c)], bb, r, c) * kc;
+    }
   }
+  if (b >= nb) return;
   const int dn = diag_node[b];
   if (dn >= 0) {
     const double M = mass[dn] * mc;  // M (1 + h alpha_k)
@@ -315,20 +385,20 @@ __global__ void fem_rhs(int N, int T, const int *__restrict__ ptr, const int *__
                         const double *__restrict__ v, const double *__restrict__ x1, double g0, double g1,
                         double g2, double h, int damp, double alpha_k, double alpha_m,
                         double *__restrict__ b) {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
+  const int a = near_block() * blockDim.x + threadIdx.x;
   if (a >= N) return;
   double s[3] = {0.0, 0.0, 0.0};
   for (int k = ptr[a]; k < ptr[a + 1]; ++k) {
     const int code = ctr[k];
     const int t = code >> 2, I = code & 3;
-    for (int r = 0; r < 3; ++r) s[r] += elem[(size_t)t * kElemOut + 144 + I * 3 + r];
+    for (int r = 0; r < 3; ++r) s[r] += elem[(size_t)T * kRec + (size_t)t * 12 + I * 3 + r];
   }
   if (damp) {
     double kd[3] = {0.0, 0.0, 0.0};
     for (int k = ptr[a]; k < ptr[a + 1]; ++k) {
       const int code = ctr[k];
       const int t = code >> 2, I = code & 3;
-      for (int r = 0; r < 3; ++r) kd[r] += elem[(size_t)t * kElemOut + 156 + I * 3 + r];
+      for (int r = 0; r < 3; ++r) kd[r] += elem[(size_t)T * (kRec + 12) + (size_t)t * 12 + I * 3 + r];
     }
     for (int r = 0; r < 3; ++r) s[r] += kd[r] * alpha_m;
   }
@@ -411,7 +481,7 @@ struct mprgp_fem {
   size_t dev_bytes = 0;
   int4 *tets = nullptr;
   double *dinv = nullptr, *vol = nullptr, *lam_mu = nullptr, *node_mass = nullptr, *mass_rho = nullptr;
-  int *blk_ptr = nullptr, *blk_ctr = nullptr, *blk_vbase = nullptr, *blk_diag = nullptr;
+  int *blk_ptr = nullptr, *blk_ctr = nullptr, *grp_ptr = nullptr, *grp_tet = nullptr, *blk_vbase = nullptr, *blk_diag = nullptr;
   int *node_ptr = nullptr, *node_ctr = nullptr;
   double *rot = nullptr;   // per-tet rotations of the last corotational assembly
   bool rot_valid = false;
@@ -501,17 +571,30 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   const long long nb = rowptr[N];
   mprgp_matrix *A = nullptr;
   if (int rc = build_matrix(ctx, N, rowptr.data(), colidx.data(), nullptr, &A)) return rc;
-  // per-block contribution lists in tet order
+  // per-block contribution lists in tet order; the blocks of each run of
+  // kGroup by descending list length (rank: a block's place)
   auto blk_of = [&](int a, int b) {
     auto it = std::lower_bound(colidx.begin() + rowptr[a], colidx.begin() + rowptr[a + 1], b);
     return (int)(it - colidx.begin());
   };
-  std::vector<int> bcnt(nb + 1, 0), ncnt(N + 1, 0);
+  std::vector<int> bcnt(nb + 1, 0), ncnt(N + 1, 0), len(nb, 0), rank(nb);
+  std::vector<int> blk(16 * (size_t)T);  // block of each tet's node pairs
   for (int t = 0; t < T; ++t)
     for (int i = 0; i < 4; ++i) {
       ncnt[tets[4 * (size_t)t + i] + 1]++;
-      for (int j = 0; j < 4; ++j) bcnt[blk_of(tets[4 * (size_t)t + i], tets[4 * (size_t)t + j]) + 1]++;
+      for (int j = 0; j < 4; ++j)
+        len[blk[16 * (size_t)t + i * 4 + j] = blk_of(tets[4 * (size_t)t + i], tets[4 * (size_t)t + j])]++;
     }
+  for (long long b0 = 0; b0 < nb; b0 += kGroup) {
+    const int n = (int)std::min<long long>(kGroup, nb - b0);
+    int by[kGroup];
+    for (int i = 0; i < n; ++i) by[i] = (int)b0 + i;
+    std::stable_sort(by, by + n, [&](int a, int b) { return len[a] > len[b]; });
+    for (int i = 0; i < n; ++i) {
+      rank[by[i]] = (int)b0 + i;
+      bcnt[b0 + i + 1] = len[by[i]];
+    }
+  }
   for (long long b = 0; b < nb; ++b) bcnt[b + 1] += bcnt[b];
   for (int a = 0; a < N; ++a) ncnt[a + 1] += ncnt[a];
   std::vector<int> bctr(bcnt[nb]), nctr(ncnt[N]);
@@ -519,10 +602,27 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
     std::vector<int> bf(bcnt.begin(), bcnt.end() - 1), nf(ncnt.begin(), ncnt.end() - 1);
     for (int t = 0; t < T; ++t)
       for (int i = 0; i < 4; ++i) {
-        int a = tets[4 * (size_t)t + i];
-        nctr[nf[a]++] = t * 4 + i;
-        for (int j = 0; j < 4; ++j) bctr[bf[blk_of(a, tets[4 * (size_t)t + j])]++] = t * 16 + i * 4 + j;
+        nctr[nf[tets[4 * (size_t)t + i]]++] = t * 4 + i;
+        for (int j = 0; j < 4; ++j) bctr[bf[rank[blk[16 * (size_t)t + i * 4 + j]]]++] = t * 16 + i * 4 + j;
       }
+  }
+  // each run's tets, ascending, and the contributions by place in that list
+  std::vector<int> gptr(1, 0), gtet, place(T, -1);
+  for (long long b0 = 0; b0 < nb; b0 += kGroup) {
+    const int k0 = bcnt[b0], k1 = bcnt[std::min<long long>(b0 + kGroup, nb)];
+    const size_t g0 = gtet.size();
+    for (int k = k0; k < k1; ++k) {
+      const int t = bctr[k] >> 4;
+      if (place[t] < 0) {
+        place[t] = 0;
+        gtet.push_back(t);
+      }
+    }
+    std::sort(gtet.begin() + g0, gtet.end());
+    for (size_t g = g0; g < gtet.size(); ++g) place[gtet[g]] = (int)(g - g0);
+    for (int k = k0; k < k1; ++k) bctr[k] = place[bctr[k] >> 4] * 16 + (bctr[k] & 15);
+    for (size_t g = g0; g < gtet.size(); ++g) place[gtet[g]] = -1;
+    gptr.push_back((int)gtet.size());
   }
   std::vector<int> vbase(nb), diag(nb, -1);
   for (int a = 0; a < N; ++a)
@@ -531,8 +631,8 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
       int s = (int)(std::upper_bound(A->sl_off_h.begin(), A->sl_off_h.end(), (int)slot) - A->sl_off_h.begin()) - 1;
       long long b0 = A->sl_off_h[s];
       long long l = (slot - b0) % kSlice, kk = (slot - b0) / kSlice;
-      vbase[k] = (int)(b0 * 9 + kk * 9 * kSlice + l);
-      if (colidx[k] == a) diag[k] = a;
+      vbase[rank[k]] = (int)(b0 * 9 + kk * 9 * kSlice + l);
+      if (colidx[k] == a) diag[rank[k]] = a;
     }
   std::vector<double> mass_rho(N);
   for (int a = 0; a < N; ++a) mass_rho[a] = mass[a] * density;  // FEMSystem::onDirty (FEMSystem.cpp:561-562)
@@ -544,8 +644,8 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   f->nb = nb;
   f->density = density;
   f->min_mass = *std::min_element(mass_rho.begin(), mass_rho.end());
-  size_t bytes = 256 * 17 + sizeof(int4) * T + sizeof(double) * (9 + 1 + 2 + 9) * (size_t)T +
-                 sizeof(double) * 2 * N + sizeof(int) * ((nb + 1) + bctr.size() + 2 * nb + (N + 1) + nctr.size());
+  size_t bytes = 256 * 19 + sizeof(int4) * T + sizeof(double) * (9 + 1 + 2 + 9) * (size_t)T +
+                 sizeof(double) * 2 * N + sizeof(int) * ((nb + 1) + bctr.size() + 2 * nb + (N + 1) + nctr.size() + gptr.size() + gtet.size());
   if (int rc = ctx->alloc(&f->dev, bytes)) {
     mprgp_matrix_destroy(A);
     delete f;
@@ -561,6 +661,8 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   f->mass_rho = carve<double>(p, N);
   f->blk_ptr = carve<int>(p, nb + 1);
   f->blk_ctr = carve<int>(p, bctr.size());
+  f->grp_ptr = carve<int>(p, gptr.size());
+  f->grp_tet = carve<int>(p, gtet.size());
   f->blk_vbase = carve<int>(p, nb);
   f->blk_diag = carve<int>(p, nb);
   f->node_ptr = carve<int>(p, N + 1);
@@ -575,6 +677,8 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   if (!e) e = hipMemcpyAsync(f->mass_rho, mass_rho.data(), sizeof(double) * N, hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->blk_ptr, bcnt.data(), sizeof(int) * (nb + 1), hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->blk_ctr, bctr.data(), sizeof(int) * bctr.size(), hipMemcpyHostToDevice, s);
+  if (!e) e = hipMemcpyAsync(f->grp_ptr, gptr.data(), sizeof(int) * gptr.size(), hipMemcpyHostToDevice, s);
+  if (!e) e = hipMemcpyAsync(f->grp_tet, gtet.data(), sizeof(int) * gtet.size(), hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->blk_vbase, vbase.data(), sizeof(int) * nb, hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->blk_diag, diag.data(), sizeof(int) * nb, hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->node_ptr, ncnt.data(), sizeof(int) * (N + 1), hipMemcpyHostToDevice, s);
@@ -637,8 +741,9 @@ int assemble_dev(mprgp_fem *f, int material, const double *xn, const double *vn,
                                               elem);
   MPRGP_HIP(hipGetLastError());
   if (!rhs_only) {
-    fem_blocks<<<(unsigned)((f->nb + 255) / 256), 256, 0, s>>>(f->nb, T, f->blk_ptr, f->blk_ctr, f->blk_vbase,
-                                                                f->blk_diag, f->mass_rho, mc, elem, f->A->d_val);
+    fem_blocks<<<(unsigned)((f->nb + kGroup - 1) / kGroup), kGroup, 0, s>>>(
+        f->nb, f->blk_ptr, f->blk_ctr, f->grp_ptr, f->grp_tet, f->blk_vbase, f->blk_diag, f->mass_rho, mc, kc, elem,
+        f->A->d_val);
     MPRGP_HIP(hipGetLastError());
   }
   fem_rhs<<<(N + 255) / 256, 256, 0, s>>>(N, T, f->node_ptr, f->node_ctr, f->node_mass, f->density, elem, xn,
