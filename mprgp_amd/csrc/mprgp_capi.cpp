@@ -101,6 +101,64 @@ void mprgp_ctx::release(void *p, size_t bytes) {
   in_use -= std::min(in_use, bytes);
 }
 
+double *mprgp_ctx::xfer_reserve(size_t bytes) {
+  if (bytes > mprgp::kXferMax) return nullptr;
+  if (bytes <= xfer_bytes) return h_xfer;
+  if (h_xfer) (void)hipHostFree(h_xfer);
+  h_xfer = nullptr;
+  xfer_bytes = 0;
+  size_t room = (size_t)1 << 16;
+  while (room < bytes) room *= 2;
+  if (hipHostMalloc((void **)&h_xfer, room, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    h_xfer = nullptr;
+    return nullptr;
+  }
+  xfer_bytes = room;
+  return h_xfer;
+}
+
+namespace mprgp {
+
+Transfer::Transfer(mprgp_ctx *ctx, size_t doubles)
+    : ctx_(ctx), pin_(doubles <= kXferMax / sizeof(double) ? ctx->xfer_reserve(sizeof(double) * doubles) : nullptr),
+      room_(doubles) {}
+// a call that fails half-way leaves no copy of its own behind
+Transfer::~Transfer() {
+  if (queued_) (void)hipStreamSynchronize(ctx_->stream);
+}
+int Transfer::up(const double *host, double *dev, size_t n) {
+  queued_ = true;
+  if (!pin_ || at_ + n > room_) {
+    MPRGP_HIP(hipMemcpyAsync(dev, host, sizeof(double) * n, hipMemcpyHostToDevice, ctx_->stream));
+    return MPRGP_OK;
+  }
+  std::memcpy(pin_ + at_, host, sizeof(double) * n);
+  MPRGP_HIP(launch_copy(ctx_->stream, pin_ + at_, dev, n));
+  at_ += n;
+  return MPRGP_OK;
+}
+int Transfer::down(const double *dev, double *host, size_t n) {
+  queued_ = true;
+  if (!pin_ || at_ + n > room_ || n_out_ == (int)(sizeof(out_) / sizeof(out_[0]))) {
+    MPRGP_HIP(hipMemcpyAsync(host, dev, sizeof(double) * n, hipMemcpyDeviceToHost, ctx_->stream));
+    return MPRGP_OK;
+  }
+  MPRGP_HIP(launch_copy(ctx_->stream, dev, pin_ + at_, n));
+  out_[n_out_++] = {pin_ + at_, host, n};
+  at_ += n;
+  return MPRGP_OK;
+}
+int Transfer::wait() {
+  queued_ = false;
+  MPRGP_HIP(hipStreamSynchronize(ctx_->stream));
+  for (int i = 0; i < n_out_; ++i) std::memcpy(out_[i].to, out_[i].from, sizeof(double) * out_[i].n);
+  n_out_ = 0;
+  return MPRGP_OK;
+}
+
+}  // namespace mprgp
+
 int mprgp_ctx::scratch_reserve(size_t bytes) {
   if (bytes <= scratch_bytes) return MPRGP_OK;
   release(scratch, scratch_bytes);
@@ -187,6 +245,7 @@ extern "C" void mprgp_ctx_destroy(mprgp_ctx *c) {
   c->release(c->scratch, c->scratch_bytes);
   if (c->h_running) (void)hipHostFree(c->h_running);
   if (c->h_final) (void)hipHostFree(c->h_final);
+  if (c->h_xfer) (void)hipHostFree(c->h_xfer);
   if (c->t0) (void)hipEventDestroy(c->t0);
   if (c->t1) (void)hipEventDestroy(c->t1);
   if (c->q[0]) (void)hipEventDestroy(c->q[0]);
@@ -773,21 +832,20 @@ extern "C" void mprgp_qp_destroy(mprgp_qp *q) {
 }
 
 // host node-order vector -> device internal order
-static int upload_vec(mprgp_qp *q, const double *h, double *dst) {
-  const size_t vb = sizeof(double) * 3 * q->n;
-  hipStream_t s = q->ctx->stream;
-  MPRGP_HIP(hipMemcpyAsync(q->stage, h, vb, hipMemcpyHostToDevice, s));
-  MPRGP_HIP(launch_gather_nodes(s, q->stage, dst, q->A->d_perm, q->n));
-  MPRGP_HIP(hipStreamSynchronize(s));
-  return MPRGP_OK;
+// (dst2: null, or a second place for it)
+static int upload_vec(mprgp_qp *q, const double *h, double *dst, double *dst2 = nullptr) {
+  const size_t n = 3 * (size_t)q->n;
+  Transfer T(q->ctx, n);
+  if (int rc = T.up(h, q->stage, n)) return rc;
+  MPRGP_HIP(launch_gather_nodes(q->ctx->stream, q->stage, dst, q->A->d_perm, q->n, dst2));
+  return T.wait();
 }
 static int download_vec(mprgp_qp *q, const double *src, double *h) {
-  const size_t vb = sizeof(double) * 3 * q->n;
-  hipStream_t s = q->ctx->stream;
-  MPRGP_HIP(launch_scatter_nodes(s, src, q->stage, q->A->d_perm, q->n));
-  MPRGP_HIP(hipMemcpyAsync(h, q->stage, vb, hipMemcpyDeviceToHost, s));
-  MPRGP_HIP(hipStreamSynchronize(s));
-  return MPRGP_OK;
+  const size_t n = 3 * (size_t)q->n;
+  Transfer T(q->ctx, n);
+  MPRGP_HIP(launch_scatter_nodes(q->ctx->stream, src, q->stage, q->A->d_perm, q->n));
+  if (int rc = T.down(q->stage, h, n)) return rc;
+  return T.wait();
 }
 
 static int check_finite(const double *v, size_t n, const char *what) {
@@ -816,10 +874,7 @@ extern "C" int mprgp_qp_set_x(mprgp_qp *q, const double *x) {
   MPRGP_NOT_BUSY(q);
   MPRGP_HIP(hipSetDevice(q->ctx->device));
   std::lock_guard<std::recursive_mutex> lk_(q->ctx->mu);
-  int rc = upload_vec(q, x, q->x0);
-  if (rc) return rc;
-  MPRGP_HIP(hipMemcpyAsync(q->x, q->x0, sizeof(double) * 3 * q->n, hipMemcpyDeviceToDevice, q->ctx->stream));
-  MPRGP_HIP(hipStreamSynchronize(q->ctx->stream));
+  if (int rc = upload_vec(q, x, q->x0, q->x)) return rc;
   q->has_x = true;
   return MPRGP_OK;
   MPRGP_CATCH
@@ -1050,10 +1105,11 @@ static int projector_call(mprgp_qp *q, int op, const double *a, const double *b,
   if (int rc = ctx->scratch_reserve(sizeof(double) * (5 * n + blocks + 1) + 1024)) return rc;
   double *ua = (double *)ctx->scratch, *ub = ua + n, *ia = ub + n, *ib = ia + n, *io = ib + n;
   double *part = io + n, *res = part + blocks;
-  MPRGP_HIP(hipMemcpyAsync(ua, a, sizeof(double) * n, hipMemcpyHostToDevice, s));
+  Transfer T(ctx, (b ? 2 : 1) * n + (out ? n : 0) + 1);
+  if (int rc = T.up(a, ua, n)) return rc;
   MPRGP_HIP(launch_gather_nodes(s, ua, ia, q->A->d_perm, N));
   if (b) {
-    MPRGP_HIP(hipMemcpyAsync(ub, b, sizeof(double) * n, hipMemcpyHostToDevice, s));
+    if (int rc = T.up(b, ub, n)) return rc;
     MPRGP_HIP(launch_gather_nodes(s, ub, ib, q->A->d_perm, N));
   }
   if (op == PJ_PRECOND) MPRGP_HIP(launch_setup_rows(s, q->A->d_dinv, q->cn, q->cf, q->cs, N));
@@ -1075,11 +1131,12 @@ static int projector_call(mprgp_qp *q, int op, const double *a, const double *b,
   MPRGP_HIP(launch_projector(s, g, res));
   if (out) {
     MPRGP_HIP(launch_scatter_nodes(s, io, ua, q->A->d_perm, N));
-    MPRGP_HIP(hipMemcpyAsync(out, ua, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+    if (int rc = T.down(ua, out, n)) return rc;
   }
   double r = 0.0;
-  if (result) MPRGP_HIP(hipMemcpyAsync(&r, res, sizeof(double), hipMemcpyDeviceToHost, s));
-  MPRGP_HIP(hipStreamSynchronize(s));
+  if (result)
+    if (int rc = T.down(res, &r, 1)) return rc;
+  if (int rc = T.wait()) return rc;
   if (result) *result = N > 0 ? r : (op == PJ_STEP_LIMIT ? kDblMax : 0.0);
   return MPRGP_OK;
 }

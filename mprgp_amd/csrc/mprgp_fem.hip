@@ -835,10 +835,10 @@ extern "C" int mprgp_fem_set_state(mprgp_fem *f, const double *x, const double *
     f->x1 = f->vn + n;
     f->x2 = f->x1 + n;
   }
-  hipStream_t s = ctx->stream;
-  MPRGP_HIP(hipMemcpyAsync(f->xn, x, sizeof(double) * n, hipMemcpyHostToDevice, s));
-  MPRGP_HIP(hipMemcpyAsync(f->vn, v, sizeof(double) * n, hipMemcpyHostToDevice, s));
-  MPRGP_HIP(hipStreamSynchronize(s));
+  Transfer T(ctx, 2 * n);
+  if (int rc = T.up(x, f->xn, n)) return rc;
+  if (int rc = T.up(v, f->vn, n)) return rc;
+  if (int rc = T.wait()) return rc;
   f->has_state = true;
   f->step_open = false;
   return MPRGP_OK;
@@ -853,11 +853,12 @@ extern "C" int mprgp_fem_get_state(mprgp_fem *f, double *x, double *v) {
   MPRGP_HIP(hipSetDevice(ctx->device));
   std::lock_guard<std::recursive_mutex> lk_(ctx->mu);
   const size_t n = 3 * (size_t)f->N;
-  hipStream_t s = ctx->stream;
-  if (x) MPRGP_HIP(hipMemcpyAsync(x, f->xn, sizeof(double) * n, hipMemcpyDeviceToHost, s));
-  if (v) MPRGP_HIP(hipMemcpyAsync(v, f->vn, sizeof(double) * n, hipMemcpyDeviceToHost, s));
-  MPRGP_HIP(hipStreamSynchronize(s));
-  return MPRGP_OK;
+  Transfer T(ctx, 2 * n);
+  if (x)
+    if (int rc = T.down(f->xn, x, n)) return rc;
+  if (v)
+    if (int rc = T.down(f->vn, v, n)) return rc;
+  return T.wait();
   MPRGP_CATCH
 }
 
@@ -963,8 +964,9 @@ extern "C" int mprgp_fem_advance(mprgp_fem *f, mprgp_qp *qp, const mprgp_step_pa
     MPRGP_HIP(launch_scatter_nodes(s, qp->x, f->x2, f->A->d_perm, N));
     if (int rc = ctx->scratch_reserve(sizeof(double) * (kMaxParts + 1))) return rc;
     MPRGP_HIP(launch_max_abs_diff(s, f->x2, f->x1, n, (double *)ctx->scratch));
-    MPRGP_HIP(hipMemcpyAsync(&st.delta, ctx->scratch, sizeof(double), hipMemcpyDeviceToHost, s));
-    MPRGP_HIP(hipStreamSynchronize(s));
+    Transfer T(ctx, 1);
+    if (int rc = T.down((const double *)ctx->scratch, &st.delta, 1)) return rc;
+    if (int rc = T.wait()) return rc;
     std::swap(f->x1, f->x2);  // x1 = the new iterate
     if (st.delta < sp->newton_eps) break;
   }

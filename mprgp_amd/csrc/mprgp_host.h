@@ -86,7 +86,10 @@ hipError_t launch_power_start(hipStream_t s, double *out, size_t n, double nr);
 hipError_t launch_step(int ts, int grid, hipStream_t s, const QpDev *qps, const Tile *tiles,
                        int *running, int parity, bool mixed, int variant = kStepCached, int spw = 1,
                        bool c16 = false);
-hipError_t launch_gather_nodes(hipStream_t s, const double *in, double *out, const int *perm, int n);
+// out2: null, or a second place for the same values
+hipError_t launch_gather_nodes(hipStream_t s, const double *in, double *out, const int *perm, int n,
+                               double *out2 = nullptr);
+hipError_t launch_copy(hipStream_t s, const double *in, double *out, size_t n);
 // setup_rows for `count` QPs of a device QpDev table (count <= 65535)
 hipError_t launch_setup_rows_batch(hipStream_t s, const QpDev *qps, int count, int max_nodes);
 // the two state copies of n QPs: staging [i][2] <-> each QP's own (ptr[i])
@@ -222,10 +225,51 @@ struct mprgp_ctx {
   void *scratch = nullptr;
   size_t scratch_bytes = 0;
   int scratch_reserve(size_t bytes);
+  // pinned memory that one call's host vectors move through (Transfer);
+  // serialised by `mu`, idle between calls
+  double *h_xfer = nullptr;
+  size_t xfer_bytes = 0;
+  double *xfer_reserve(size_t bytes);
 
   int alloc(void **p, size_t bytes);
   void release(void *p, size_t bytes);
 };
+
+namespace mprgp {
+
+// The host vectors of one call on a context (its lock held): up() and down()
+// queue copies, wait() waits for the stream once and hands out what came
+// down.  Vectors go through the context's pinned memory, which a kernel reads
+// and writes (a 12 KB vector to the host 15 us, with its wait; 28 us as a copy
+// to pageable memory; 46 KB 17 and 42, 164 KB 21 and 90, 1 MB 69 and 81 us;
+// copies queued on pinned memory lie between).  Calls of more than kXferMax
+// bytes copy from and to the caller's memory, where the difference is gone
+// (3.5 MB: 209 and 220 us), as they do where no pinned memory is to be had.
+constexpr size_t kXferMax = (size_t)4 << 20;
+class Transfer {
+ public:
+  Transfer(mprgp_ctx *ctx, size_t doubles);
+  ~Transfer();
+  Transfer(const Transfer &) = delete;
+  Transfer &operator=(const Transfer &) = delete;
+  int up(const double *host, double *dev, size_t n);
+  int down(const double *dev, double *host, size_t n);
+  int wait();
+
+ private:
+  mprgp_ctx *ctx_;
+  double *pin_;
+  size_t at_ = 0, room_;
+  bool queued_ = false;
+  int n_out_ = 0;
+  struct Out {
+    const double *from;
+    double *to;
+    size_t n;
+  } out_[4];
+};
+
+}  // namespace mprgp
 
 struct mprgp_matrix {
   mprgp_ctx *ctx = nullptr;

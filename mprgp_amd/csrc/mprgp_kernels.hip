@@ -1490,13 +1490,19 @@ __global__ void __launch_bounds__(TS * kSlice, UB == kUnroll ? MPRGP_STEP_MIN_WA
 
 // out[i] = in[perm[i]]: user node order -> internal order.
 __global__ void gather_nodes(const double *__restrict__ in, double *__restrict__ out,
-                             const int *__restrict__ perm, int n_nodes) {
+                             const int *__restrict__ perm, int n_nodes, double *__restrict__ out2) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_nodes) return;
   int o = perm[i];
-  out[3 * (size_t)i + 0] = in[3 * (size_t)o + 0];
-  out[3 * (size_t)i + 1] = in[3 * (size_t)o + 1];
-  out[3 * (size_t)i + 2] = in[3 * (size_t)o + 2];
+  for (int k = 0; k < 3; ++k) {
+    const double v = in[3 * (size_t)o + k];
+    out[3 * (size_t)i + k] = v;
+    if (out2) out2[3 * (size_t)i + k] = v;
+  }
+}
+__global__ void copy_doubles(const double *__restrict__ in, double *__restrict__ out, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = in[i];
 }
 // out[perm[i]] = in[i]: internal order -> user node order.
 __global__ void scatter_nodes(const double *__restrict__ in, double *__restrict__ out,
@@ -1925,9 +1931,15 @@ hipError_t launch_gather_states(hipStream_t s, QpState *const *src, QpState *dst
   gather_states<<<n, 64, 0, s>>>(reinterpret_cast<const double2 *const *>(src), reinterpret_cast<double2 *>(dst), n);
   return hipGetLastError();
 }
-hipError_t launch_gather_nodes(hipStream_t s, const double *in, double *out, const int *perm, int n) {
+hipError_t launch_copy(hipStream_t s, const double *in, double *out, size_t n) {
+  if (n == 0) return hipSuccess;
+  if (n > ((size_t)1 << 31)) return hipErrorInvalidValue;
+  copy_doubles<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(in, out, n);
+  return hipGetLastError();
+}
+hipError_t launch_gather_nodes(hipStream_t s, const double *in, double *out, const int *perm, int n, double *out2) {
   if (n <= 0) return hipSuccess;
-  gather_nodes<<<(n + 255) / 256, 256, 0, s>>>(in, out, perm, n);
+  gather_nodes<<<(n + 255) / 256, 256, 0, s>>>(in, out, perm, n, out2);
   return hipGetLastError();
 }
 hipError_t launch_scatter_nodes(hipStream_t s, const double *in, double *out, const int *perm, int n) {
