@@ -85,8 +85,8 @@ typedef struct {
   int max_refine;      /* MIXED: outer refinement sweeps (0 = default 8)             */
   int tail_tiles;      /* launches of at most this many tiles run the step kernel's  */
                        /* tail form (same results); 0 = 256, one per CU              */
-  int xcd_layout;      /* workgroups over the 8 XCDs (same results): 0 runs of 4     */
-                       /* tiles rotating, 1 one contiguous chunk of each QP per XCD  */
+  int xcd_layout;      /* workgroups over the 8 XCDs (same results): 0 runs of 4 to  */
+                       /* 32 tiles rotating, 1 one contiguous chunk of each QP per XCD  */
   int slices_per_wave; /* SELL slices (64 rows) each wavefront streams per launch:   */
                        /* 0 or 1, or 2 (rows per wavefront = 64 x this; a tile is    */
                        /* tiles x this slices; like tiles, it groups the sums)       */

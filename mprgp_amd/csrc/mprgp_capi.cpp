@@ -1425,23 +1425,20 @@ void append_tiles(int slot, const mprgp_qp *q, int span, std::vector<Tile> &tile
 }
 
 // Workgroups per launch: one per tile, rounded up to a power of two so that
-// few distinct graphs get captured.
+// few distinct graphs get captured; up to kXcdCus tiles an XCD takes all of
+// them (the workgroups of unused slots exit at once: 256 against 64 cost less
+// than the launch times differ).
 int round_grid(int n_tiles) {
   int g = 64;
-  while (g < n_tiles) g *= 2;
+  while (g < n_tiles || (g < kXcds * kXcdCus && g < kXcds * n_tiles)) g *= 2;
   return g;
 }
 
 // The table a launch of `grid` workgroups reads, one slot per workgroup;
 // unused slots hold qp = -1.  Workgroups go to the 8 XCDs of the MI355X
 // round-robin (workgroup b to XCD b % 8), each XCD with its own L2: runs of
-// kXcdRun consecutive tiles (neighbouring rows, which gather from each
-// other) go to one XCD, and the runs rotate over the XCDs so that every XCD
-// samples every QP.  On the 256-QP batch, runs of 4 measured 0.7% faster
-// than single tiles, runs of 16 1% slower, and whole QPs per XCD 6% slower:
-// per-QP work differs by op and one XCD's share then sets the launch time.
-constexpr int kXcds = 8;
-constexpr int kXcdRun = 4;
+// xcd_run consecutive tiles (neighbouring rows, which gather from each
+// other) go to one XCD, and the runs rotate over the XCDs.
 // layout 1 (per-QP chunks): each QP's tiles split into kXcds contiguous
 // chunks, one per XCD, so an XCD gathers from one contiguous part of each
 // QP's vectors; chunk sizes differ by at most one tile, the larger ones going
@@ -1478,9 +1475,9 @@ static bool layout_chunks(const std::vector<Tile> &tiles, int grid, Tile *table)
 void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int layout) {
   if (layout == 1 && layout_chunks(tiles, grid, table)) return;
   const int n = (int)tiles.size();
-  // grid is a power of two >= 64, so c * kXcds divides it and every slot
-  // below lands inside the table
-  const int c = std::min(kXcdRun, grid / kXcds);
+  // grid and the run are powers of two, grid at least 64, so c * kXcds divides
+  // it and every slot below lands inside the table
+  const int c = xcd_run(n, grid);
   for (int b = 0; b < grid; ++b) table[b] = Tile{nullptr, nullptr, -1, 0, 0, 0, 0, 0};
   for (int i = 0; i < n; ++i) {
     const int xcd = (i / c) % kXcds, pos = (i / (c * kXcds)) * c + i % c;

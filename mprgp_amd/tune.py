@@ -48,7 +48,7 @@ TAIL_CANDIDATES = [0, 64, 128, 512, 1024, 2048]
 LAYOUT_CANDIDATES = [0, 1]
 
 # Bumped whenever the step kernel changes in a way that moves the best shape.
-CACHE_VERSION = 7
+CACHE_VERSION = 8
 
 
 def cache_path():
