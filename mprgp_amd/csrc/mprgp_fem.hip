@@ -556,6 +556,11 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
     for (int j = 0; j < 4; ++j) mass[tets[4 * (size_t)t + j]] += vol[t] / 4.0;  // FEMMesh.cpp:507-509
   // node adjacency -> block pattern (sorted neighbours, self included)
   std::vector<std::vector<int>> nbr(N);
+  {
+    std::vector<int> of(N, 0);  // tets of each node
+    for (int v : tets) of[v]++;
+    for (int a = 0; a < N; ++a) nbr[a].reserve(4 * (size_t)of[a] + 1);
+  }
   for (int t = 0; t < T; ++t)
     for (int i = 0; i < 4; ++i)
       for (int j = 0; j < 4; ++j) nbr[tets[4 * (size_t)t + i]].push_back(tets[4 * (size_t)t + j]);
