@@ -101,28 +101,10 @@ void mprgp_ctx::release(void *p, size_t bytes) {
   in_use -= std::min(in_use, bytes);
 }
 
-double *mprgp_ctx::xfer_reserve(size_t bytes) {
-  if (bytes > mprgp::kXferMax) return nullptr;
-  if (bytes <= xfer_bytes) return h_xfer;
-  if (h_xfer) (void)hipHostFree(h_xfer);
-  h_xfer = nullptr;
-  xfer_bytes = 0;
-  size_t room = (size_t)1 << 16;
-  while (room < bytes) room *= 2;
-  if (hipHostMalloc((void **)&h_xfer, room, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    h_xfer = nullptr;
-    return nullptr;
-  }
-  xfer_bytes = room;
-  return h_xfer;
-}
-
 namespace mprgp {
 
 Transfer::Transfer(mprgp_ctx *ctx, size_t doubles)
-    : ctx_(ctx), pin_(doubles <= kXferMax / sizeof(double) ? ctx->xfer_reserve(sizeof(double) * doubles) : nullptr),
-      room_(doubles) {}
+    : ctx_(ctx), pin_(doubles <= kXferMax / sizeof(double) ? ctx->h_xfer : nullptr), room_(doubles) {}
 // a call that fails half-way leaves no copy of its own behind
 Transfer::~Transfer() {
   if (queued_) (void)hipStreamSynchronize(ctx_->stream);
@@ -224,6 +206,11 @@ extern "C" int mprgp_ctx_create(int device, size_t hbm_budget_bytes, mprgp_ctx *
   if (e != hipSuccess) {
     mprgp_ctx_destroy(c);
     return fail(MPRGP_EHIP, "context setup failed: %s", hipGetErrorString(e));
+  }
+  // without it the host vectors are copied from where they are
+  if (hipHostMalloc((void **)&c->h_xfer, kXferMax, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    c->h_xfer = nullptr;
   }
   int rc = c->tab.init(c);
   if (!rc) rc = noalloc_setup(device);

@@ -1,8 +1,8 @@
 """Host vectors of one call through the context's pinned memory: round trips
-and projections are exact at the sizes where that memory is first made (64
-KB), grown, and given up for plain copies (4 MB a call: one vector of 174,762
-nodes; a projection's two vectors and its sum, 87,380 nodes), each after
-larger and smaller calls on the same context."""
+and projections are exact for small calls and at the sizes where that memory
+is given up for plain copies (4 MB a call: one vector of 174,762 nodes; a
+projection's two vectors and its sum, 87,380 nodes), each after larger and
+smaller calls on the same context."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -23,7 +23,7 @@ def test_vectors_arrive_whole(sizes):
     ctx = M.Context(0)
     qps = [body(ctx, n) for n in sizes]
     rng = np.random.default_rng(0)
-    for _ in range(2):  # the second pass finds the memory that the largest call left
+    for _ in range(2):
         for q, n in zip(qps, sizes):
             x, b = rng.standard_normal(3 * n), rng.standard_normal(3 * n)
             q.set_x(x)
