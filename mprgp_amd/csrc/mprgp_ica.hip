@@ -537,11 +537,11 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
     }
     lo_ptr[t + 1] = (int)lo_slot.size();
   }
-  size_t n_lo = lo_slot.size();
+  const size_t n_lo = lo_slot.size();
   // the ring sweep's levels, if every column a level reads is within kRing
   // positions of the level's end and the padded blocks stay few
   std::vector<SweepLevel> lvl(n_levels);
-  std::vector<int> lo_cnt(nn), lo_ring;
+  std::vector<int> lo_cnt(nn), ring_slot, lo_ring;  // the padded blocks' SELL slots and ring slots
   bool use_ring = true;
   int ring_threads = 64;
   size_t n_pad = 0;
@@ -565,30 +565,36 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
     for (const SweepLevel &L : lvl) widest = std::max(widest, L.count);
     n_pad += widest + kAhead;
     ring_threads = std::min(kRingThreads, (4 * widest + 63) / 64 * 64);
-    std::vector<int> slot_p(n_pad, -1);
+    ring_slot.assign(n_pad, -1);
     lo_ring.assign(n_pad, 0);
     for (const SweepLevel &L : lvl)
       for (int qn = 0; qn < L.count; ++qn)
         for (int b = 0; b < lo_cnt[L.t0 + qn]; ++b) {
           const size_t e = lo_ptr[L.t0 + qn] + b;
-          slot_p[(size_t)L.base + (size_t)b * L.count + qn] = lo_slot[e];
+          ring_slot[(size_t)L.base + (size_t)b * L.count + qn] = lo_slot[e];
           lo_ring[(size_t)L.base + (size_t)qn * L.blocks + b] = 3 * (pos[lo_col[e]] % kRing);
         }
-    lo_slot.swap(slot_p);
-    lo_col.swap(lo_ring);  // the column list the kernel reads: ring slots
-    n_lo = n_pad;
   }
 
   // device block: Da^-1, levels, the lower blocks and their values, J and
-  // J^T, J u, lambda, dot partials
+  // J^T, J u, lambda, dot partials.  The ring sweep's, with up to three times
+  // the blocks and a second Da^-1, is the larger; where it is refused, the
+  // sweep that reads x from memory takes its place.
   const size_t parts = ((size_t)n + 255) / 256 + 1;
-  const size_t bytes = sizeof(double) * ((use_ring ? 18 : 9) * (size_t)nn + 9 * n_lo + 2 * (size_t)nnz + 2 * (size_t)m +
-                                         parts + 8) +
-                       sizeof(int) * ((size_t)n_levels + 1 + 3 * ((size_t)nn + 1) + 2 * n_lo + 4 * (size_t)n_levels +
-                                      (size_t)m + 1 + 2 * (size_t)nnz + (size_t)n + 1) +
-                       1024;
+  const size_t common = sizeof(double) * (2 * (size_t)nnz + 2 * (size_t)m + parts + 8) +
+                        sizeof(int) * ((size_t)m + 1 + 2 * (size_t)nnz + (size_t)n + 1) + 1024;
+  size_t bytes = common + sizeof(double) * (18 * (size_t)nn + 9 * n_pad) +
+                 sizeof(int) * (3 * (size_t)nn + 1 + 2 * n_pad) + sizeof(SweepLevel) * (size_t)n_levels;
   void *blk = nullptr;
-  if (int rc = ctx->alloc(&blk, bytes)) return rc;
+  use_ring = use_ring && ctx->alloc(&blk, bytes) == MPRGP_OK;
+  if (!use_ring) {
+    bytes = common + sizeof(double) * (9 * (size_t)nn + 9 * n_lo) +
+            sizeof(int) * ((size_t)n_levels + 1 + 2 * (size_t)nn + 1 + 2 * n_lo);
+    if (int rc = ctx->alloc(&blk, bytes)) return rc;
+  }
+  // the blocks as the chosen sweep reads them
+  const size_t n_blk = use_ring ? n_pad : n_lo;
+  const std::vector<int> &blk_slot = use_ring ? ring_slot : lo_slot, &blk_col = use_ring ? lo_ring : lo_col;
   struct Release {  // on every exit: the stream's work on the block ends first
     mprgp_ctx *c;
     void *p;
@@ -610,15 +616,15 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
   double *d_jx = (double *)carve(sizeof(double) * (m + 1));
   double *d_lam = (double *)carve(sizeof(double) * (m + 1));
   double *d_part = (double *)carve(sizeof(double) * parts);
-  int *d_lvl_ptr = (int *)carve(sizeof(int) * (n_levels + 1));
+  int *d_lvl_ptr = use_ring ? nullptr : (int *)carve(sizeof(int) * (n_levels + 1));
   int *d_lvl_node = (int *)carve(sizeof(int) * (size_t)nn);
-  double *d_lo_val = (double *)carve(sizeof(double) * 9 * n_lo);
+  double *d_lo_val = (double *)carve(sizeof(double) * 9 * n_blk);
   int *d_lo_ptr = (int *)carve(sizeof(int) * ((size_t)nn + 1));
-  int *d_lo_slot = (int *)carve(sizeof(int) * n_lo);
-  int *d_lo_col = (int *)carve(sizeof(int) * n_lo);
+  int *d_lo_slot = (int *)carve(sizeof(int) * n_blk);
+  int *d_lo_col = (int *)carve(sizeof(int) * n_blk);
   double *d_dinv_t = use_ring ? (double *)carve(sizeof(double) * 9 * (size_t)nn) : nullptr;
-  SweepLevel *d_lvl = (SweepLevel *)carve(sizeof(SweepLevel) * (size_t)n_levels);
-  int *d_pos = (int *)carve(sizeof(int) * (size_t)nn);
+  SweepLevel *d_lvl = use_ring ? (SweepLevel *)carve(sizeof(SweepLevel) * (size_t)n_levels) : nullptr;
+  int *d_pos = use_ring ? (int *)carve(sizeof(int) * (size_t)nn) : nullptr;
   int *d_jp = (int *)carve(sizeof(int) * (m + 1));
   int *d_jc = (int *)carve(sizeof(int) * nnz);
   int *d_tp = (int *)carve(sizeof(int) * (n + 1));
@@ -631,7 +637,6 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
     MPRGP_HIP(hipMemcpyAsync(d_tv, Ri.tv.data(), sizeof(double) * nnz, hipMemcpyHostToDevice, s));
   }
   MPRGP_HIP(hipMemcpyAsync(d_tp, Ri.tptr.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, s));
-  MPRGP_HIP(hipMemcpyAsync(d_lvl_ptr, lvl_ptr.data(), sizeof(int) * (n_levels + 1), hipMemcpyHostToDevice, s));
   MPRGP_HIP(hipMemcpyAsync(d_lvl_node, lvl_node.data(), sizeof(int) * (size_t)nn, hipMemcpyHostToDevice, s));
   if (use_ring) {
     MPRGP_HIP(hipMemcpyAsync(d_lo_ptr, lo_cnt.data(), sizeof(int) * (size_t)nn, hipMemcpyHostToDevice, s));
@@ -640,11 +645,12 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
     MPRGP_HIP(hipFuncSetAttribute((const void *)ica_sweep_ring, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   3 * kRing * (int)sizeof(double)));
   } else {
+    MPRGP_HIP(hipMemcpyAsync(d_lvl_ptr, lvl_ptr.data(), sizeof(int) * (n_levels + 1), hipMemcpyHostToDevice, s));
     MPRGP_HIP(hipMemcpyAsync(d_lo_ptr, lo_ptr.data(), sizeof(int) * ((size_t)nn + 1), hipMemcpyHostToDevice, s));
   }
-  if (n_lo > 0) {
-    MPRGP_HIP(hipMemcpyAsync(d_lo_slot, lo_slot.data(), sizeof(int) * n_lo, hipMemcpyHostToDevice, s));
-    MPRGP_HIP(hipMemcpyAsync(d_lo_col, lo_col.data(), sizeof(int) * n_lo, hipMemcpyHostToDevice, s));
+  if (n_blk > 0) {
+    MPRGP_HIP(hipMemcpyAsync(d_lo_slot, blk_slot.data(), sizeof(int) * n_blk, hipMemcpyHostToDevice, s));
+    MPRGP_HIP(hipMemcpyAsync(d_lo_col, blk_col.data(), sizeof(int) * n_blk, hipMemcpyHostToDevice, s));
   }
   const int blocks = (nn + 255) / 256;
   if (nn > 0) {
@@ -655,11 +661,10 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
     ica_order_dinv<<<(9 * nn + 255) / 256, 256, 0, s>>>(d_dinv, d_lvl_node, nn, d_dinv_t);
     MPRGP_HIP(hipGetLastError());
   }
-  if (n_lo > 0 && use_ring) {
-    ica_ring_vals<<<(unsigned)((n_lo + 255) / 256), 256, 0, s>>>(A->d_val, d_lo_slot, (int)n_lo, d_lo_val);
-    MPRGP_HIP(hipGetLastError());
-  } else if (n_lo > 0) {
-    ica_lower_vals<<<(unsigned)((n_lo + 255) / 256), 256, 0, s>>>(A->d_val, d_lo_slot, (int)n_lo, d_lo_val);
+  if (n_blk > 0) {
+    const unsigned grid = (unsigned)((n_blk + 255) / 256);
+    if (use_ring) ica_ring_vals<<<grid, 256, 0, s>>>(A->d_val, d_lo_slot, (int)n_blk, d_lo_val);
+    else ica_lower_vals<<<grid, 256, 0, s>>>(A->d_val, d_lo_slot, (int)n_blk, d_lo_val);
     MPRGP_HIP(hipGetLastError());
   }
   // B = J Da^-1 J^T on the host, from the inverse blocks in user order
@@ -680,20 +685,23 @@ extern "C" int mprgp_ica_solve(mprgp_qp *q, int m, const int *j_ptr, const int *
   }
   double *u = q->z, *jtl = q->phi, *rh = q->beta, *e = q->ap;
   const double *x_c = q->x;
-  // pinned: J u and the residual as read back (d_jx, m + 1 doubles), lambda
+  // J u and the residual as read back (d_jx, m + 1 doubles), lambda: pinned
+  // where that is to be had.  Every iteration waits for the readback before
+  // lambda is written again.
   struct Pinned {
     double *p = nullptr;
     ~Pinned() {
       if (p) (void)hipHostFree(p);
     }
   } pin;
+  std::vector<double> pageable;
   if (hipHostMalloc((void **)&pin.p, sizeof(double) * (2 * (size_t)m + 1), hipHostMallocDefault) != hipSuccess) {
     pin.p = nullptr;
     (void)hipGetLastError();
-    return fail(MPRGP_ENOMEM, "pinned staging of %d multipliers", m);
+    pageable.resize(2 * (size_t)m + 1);
   }
-  double *h_jx = pin.p, *h_lam = pin.p + m + 1, *d_r2 = d_jx + m;
-  Release drain_{ctx, nullptr, 0};  // before the pinned block goes: an upload from it may be queued
+  double *h_jx = pin.p ? pin.p : pageable.data(), *h_lam = h_jx + m + 1, *d_r2 = d_jx + m;
+  Release drain_{ctx, nullptr, 0};  // before that memory goes: an upload from it may be queued
   MPRGP_HIP(hipMemsetAsync(jtl, 0, sizeof(double) * n, s));
   MPRGP_HIP(hipMemsetAsync(d_jx, 0, sizeof(double) * ((size_t)m + 1), s));
   MPRGP_HIP(hipEventRecord(ctx->t0, s));

@@ -1,0 +1,70 @@
+"""Solves that prefer a form with more device memory still run, with the same
+results, where the context's budget holds only the form with less."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import mprgp_amd as M
+from mprgp_amd import problems
+from tests.common import scene_qp
+
+pytestmark = pytest.mark.gpu
+
+
+def beam():
+    sc = problems.beam_scene("b", 12, 4, 4, seed=3, tol=1e-8)
+    A, b, node, normal, c, x0 = scene_qp(sc)
+    Jc, cc = problems.self_contact_rows(sc, np.random.default_rng(2), 6)
+    return A, b, sp.vstack([problems.rows_to_J(node, normal, sc.n_nodes), Jc]).tocsr(), np.concatenate([c, cc]), x0
+
+
+def on_budget(A, b, x0, call, extra=None):
+    """call(qp) on a context of its own; extra: bytes allowed beyond the matrix and the QP."""
+    ctx = M.Context(0)
+    try:
+        q = ctx.matrix_csr(A).qp()
+        used = ctx.memory()[0]
+    finally:
+        ctx.close()
+    ctx = M.Context(0, hbm_budget=0 if extra is None else used + extra)
+    try:
+        q = ctx.matrix_csr(A).qp()
+        q.set_rhs(b)
+        q.set_x(x0)
+        out = call(q)
+        return out, q.get_x()
+    finally:
+        ctx.close()
+
+
+def lower_levels(A):
+    """Blocks below the diagonal and dependency levels of the forward sweep."""
+    P = sp.csr_matrix(A).tobsr((3, 3))
+    level = np.zeros(A.shape[0] // 3, int)
+    n_lo = 0
+    for i in range(level.size):
+        lo = P.indices[P.indptr[i]:P.indptr[i + 1]]
+        lo = lo[lo < i]
+        n_lo += lo.size
+        level[i] = level[lo].max() + 1 if lo.size else 0
+    return n_lo, level.max() + 1
+
+
+def test_ica_without_room_for_the_ring(ctx):
+    A, b, J, c, x0 = beam()
+    n, nn, m, nnz = A.shape[0], A.shape[0] // 3, J.shape[0], J.nnz
+    n_lo, levels = lower_levels(A)
+    parts = (n + 255) // 256 + 1
+    least = 8 * (9 * nn + 9 * n_lo + 2 * nnz + 2 * m + parts + 8) + \
+        4 * (levels + 1 + 2 * nn + 1 + 2 * n_lo + m + 1 + 2 * nnz + n + 1) + 1024
+
+    def call(q):
+        rc, st, lam, sweeps = M.ica_solve(q, J, c, tol=1e-6, max_it=30, gs_max_it=20, gs_tol=1e-8)
+        return rc, st["iterations"], st["residual"], sweeps, lam.tobytes()
+    free, xf = on_budget(A, b, x0, call)
+    tight, xt = on_budget(A, b, x0, call, least)
+    assert tight == free
+    np.testing.assert_array_equal(xt, xf)
+    with pytest.raises(M.MprgpError) as e:
+        on_budget(A, b, x0, call, least - 2048)
+    assert e.value.code == -7
