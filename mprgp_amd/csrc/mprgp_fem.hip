@@ -577,57 +577,63 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   mprgp_matrix *A = nullptr;
   if (int rc = build_matrix(ctx, N, rowptr.data(), colidx.data(), nullptr, &A)) return rc;
   // per-block contribution lists in tet order; the blocks of each run of
-  // kGroup by descending list length (rank: a block's place)
+  // kGroup by descending list length (rank: a block's place; lists of kLong
+  // and more count as equal), and each run's tets, ascending, by whose place
+  // in that list (the run's last tet so far) a contribution names its tet.
+  // Filled tet by tet, so nothing is sorted: sorting the blocks and the tets
+  // of each run made a body of 44,541 nodes 74 ms instead of 64, one of 15,975 20.4 instead of 17.3.
   auto blk_of = [&](int a, int b) {
     auto it = std::lower_bound(colidx.begin() + rowptr[a], colidx.begin() + rowptr[a + 1], b);
     return (int)(it - colidx.begin());
   };
-  std::vector<int> bcnt(nb + 1, 0), ncnt(N + 1, 0), len(nb, 0), rank(nb);
+  constexpr int kLong = 63;
+  const int runs = (int)((nb + kGroup - 1) / kGroup);
+  std::vector<int> bcnt(nb + 1, 0), ncnt(N + 1, 0), len(nb, 0), rank(nb), gptr(runs + 1, 0), last(runs, -1);
   std::vector<int> blk(16 * (size_t)T);  // block of each tet's node pairs
   for (int t = 0; t < T; ++t)
     for (int i = 0; i < 4; ++i) {
       ncnt[tets[4 * (size_t)t + i] + 1]++;
-      for (int j = 0; j < 4; ++j)
-        len[blk[16 * (size_t)t + i * 4 + j] = blk_of(tets[4 * (size_t)t + i], tets[4 * (size_t)t + j])]++;
+      for (int j = 0; j < 4; ++j) {
+        const int b = blk_of(tets[4 * (size_t)t + i], tets[4 * (size_t)t + j]), g = b / kGroup;
+        blk[16 * (size_t)t + i * 4 + j] = b;
+        len[b]++;
+        if (last[g] != t) {
+          last[g] = t;
+          gptr[g + 1]++;
+        }
+      }
     }
   for (long long b0 = 0; b0 < nb; b0 += kGroup) {
     const int n = (int)std::min<long long>(kGroup, nb - b0);
-    int by[kGroup];
-    for (int i = 0; i < n; ++i) by[i] = (int)b0 + i;
-    std::stable_sort(by, by + n, [&](int a, int b) { return len[a] > len[b]; });
+    int at[kLong + 2] = {0};
+    for (int i = 0; i < n; ++i) at[kLong - std::min(len[b0 + i], kLong) + 1]++;
+    for (int k = 0; k <= kLong; ++k) at[k + 1] += at[k];
     for (int i = 0; i < n; ++i) {
-      rank[by[i]] = (int)b0 + i;
-      bcnt[b0 + i + 1] = len[by[i]];
+      const int r = at[kLong - std::min(len[b0 + i], kLong)]++;
+      rank[b0 + i] = (int)b0 + r;
+      bcnt[b0 + r + 1] = len[b0 + i];
     }
   }
   for (long long b = 0; b < nb; ++b) bcnt[b + 1] += bcnt[b];
   for (int a = 0; a < N; ++a) ncnt[a + 1] += ncnt[a];
-  std::vector<int> bctr(bcnt[nb]), nctr(ncnt[N]);
+  for (int g = 0; g < runs; ++g) gptr[g + 1] += gptr[g];
+  std::vector<int> bctr(bcnt[nb]), nctr(ncnt[N]), gtet(gptr[runs]);
   {
     std::vector<int> bf(bcnt.begin(), bcnt.end() - 1), nf(ncnt.begin(), ncnt.end() - 1);
+    std::vector<int> gf(gptr.begin(), gptr.end() - 1);
+    std::fill(last.begin(), last.end(), -1);
     for (int t = 0; t < T; ++t)
       for (int i = 0; i < 4; ++i) {
         nctr[nf[tets[4 * (size_t)t + i]]++] = t * 4 + i;
-        for (int j = 0; j < 4; ++j) bctr[bf[rank[blk[16 * (size_t)t + i * 4 + j]]]++] = t * 16 + i * 4 + j;
+        for (int j = 0; j < 4; ++j) {
+          const int b = blk[16 * (size_t)t + i * 4 + j], g = b / kGroup;
+          if (last[g] != t) {
+            last[g] = t;
+            gtet[gf[g]++] = t;
+          }
+          bctr[bf[rank[b]]++] = (gf[g] - 1 - gptr[g]) * 16 + i * 4 + j;
+        }
       }
-  }
-  // each run's tets, ascending, and the contributions by place in that list
-  std::vector<int> gptr(1, 0), gtet, place(T, -1);
-  for (long long b0 = 0; b0 < nb; b0 += kGroup) {
-    const int k0 = bcnt[b0], k1 = bcnt[std::min<long long>(b0 + kGroup, nb)];
-    const size_t g0 = gtet.size();
-    for (int k = k0; k < k1; ++k) {
-      const int t = bctr[k] >> 4;
-      if (place[t] < 0) {
-        place[t] = 0;
-        gtet.push_back(t);
-      }
-    }
-    std::sort(gtet.begin() + g0, gtet.end());
-    for (size_t g = g0; g < gtet.size(); ++g) place[gtet[g]] = (int)(g - g0);
-    for (int k = k0; k < k1; ++k) bctr[k] = place[bctr[k] >> 4] * 16 + (bctr[k] & 15);
-    for (size_t g = g0; g < gtet.size(); ++g) place[gtet[g]] = -1;
-    gptr.push_back((int)gtet.size());
   }
   std::vector<int> vbase(nb), diag(nb, -1);
   for (int a = 0; a < N; ++a)
