@@ -1459,12 +1459,12 @@ static bool layout_chunks(const std::vector<Tile> &tiles, int grid, Tile *table)
   return true;
 }
 
-void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int layout) {
+void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int span, int layout) {
   if (layout == 1 && layout_chunks(tiles, grid, table)) return;
   const int n = (int)tiles.size();
   // grid and the run are powers of two, grid at least 64, so c * kXcds divides
   // it and every slot below lands inside the table
-  const int c = xcd_run(n, grid);
+  const int c = xcd_run(n, grid, span);
   for (int b = 0; b < grid; ++b) table[b] = Tile{nullptr, nullptr, -1, 0, 0, 0, 0, 0};
   for (int i = 0; i < n; ++i) {
     const int xcd = (i / c) % kXcds, pos = (i / (c * kXcds)) * c + i % c;
@@ -1677,7 +1677,7 @@ static int run_batch(mprgp_ctx *ctx, int count, mprgp_qp *const *qps, const mprg
   if (int rc = tab.ensure(count, grid)) return rc;
   if (int rc = tab.ensure_states(count)) return rc;
   const int layout = params[0].xcd_layout;
-  layout_tiles(tiles, grid, tab.h_tiles, layout);
+  layout_tiles(tiles, grid, tab.h_tiles, span, layout);
   hipStream_t s = ctx->stream;
   std::vector<QpDev> devs(count);
   QpState *states = tab.h_states;  // pinned; [i][2]
@@ -1780,7 +1780,7 @@ static int run_batch(mprgp_ctx *ctx, int count, mprgp_qp *const *qps, const mprg
         for (int i = 0; i < count; ++i)
           if (keep[i]) append_tiles(i, qps[i], span, kept);
         grid = round_grid((int)kept.size());  // <= the table's capacity: the tile count only shrinks
-        layout_tiles(kept, grid, tab.h_tiles, layout);
+        layout_tiles(kept, grid, tab.h_tiles, span, layout);
         MPRGP_HIP(hipMemcpyAsync(tab.d_tiles, tab.h_tiles, sizeof(Tile) * grid, hipMemcpyHostToDevice, s));
         in_table = live;
         shrunk_at = k;

@@ -170,20 +170,31 @@ inline bool use_col16(bool all_have, int spw) {
 void append_tiles(int slot, const mprgp_qp *q, int span, std::vector<Tile> &tiles);
 int tiles_for(int n_slices, int span);
 int round_grid(int n_tiles);
-// Tiles that stand side by side on one XCD (32 CUs, an L2 of its own).
-//   Up to a tile per CU of the card: 32, an XCD's share.  A launch then lasts
-//   as long as a lone tile, most of that waiting for what other tiles wrote,
-//   which the XCD's own L2 holds (9 tiles, 1,575 DoF: 1370 us a solve in runs
-//   of 4, 1323 in runs of 32; 31 tiles with its power method 16.7 and 15.0
-//   ms; 106 tiles 13.13 and 13.0; 112 tiles, mixed, 1800 and 1746 us).
-//   Up to 4 per CU: 16 (348 tiles 3963 us in runs of 4, 3917 in runs of 16,
-//   4047 in runs of 32; 24 QPs 5.71, 5.60 and 5.66 ms).
+// Tiles of `span` slices that stand side by side on one XCD (32 CUs, an L2 of
+// its own).
+//   Up to a tile per CU of the card: 32 slices.  A launch then lasts as long
+//   as a lone tile, most of that waiting for what other tiles wrote, which the
+//   XCD's own L2 holds (9 tiles of one slice, 1,575 DoF: 1370 us a solve in
+//   runs of 4, 1323 in runs of 32; 31 tiles with its power method 16.7 and
+//   15.0 ms; 106 tiles 13.13 and 13.0; 112 tiles, mixed, 1800 and 1746 us).
+//   More slices side by side are bound by the XCD's share of the memory rate:
+//   32 tiles on one, and 32 slices, of 15,975 nodes in tiles of 4 2,282 and
+//   1,984 us, mixed 1,465 and 1,228; of 44,541 nodes in tiles of 8 4,565 and
+//   3,748, mixed 2,056 and 1,711.
+//   Up to 4 per CU: 16 tiles, 32 slices at most (348 tiles of two slices 3963
+//   us in runs of 4, 3917 in runs of 16, 4047 in runs of 32; 24 QPs 5.71, 5.60
+//   and 5.66 ms).
 //   Beyond: 4, so that every XCD samples every QP: per-QP work differs by op
 //   and one XCD's share sets the launch time (256 QPs: runs of 4 0.7% faster
 //   than single tiles, runs of 16 1% slower, whole QPs per XCD 6% slower).
+// At least 4, and what the launch's slots hold.
 constexpr int kXcds = 8, kXcdCus = 32;
-inline int xcd_run(int n_tiles, int grid) {
-  const int run = n_tiles <= kXcds * kXcdCus ? kXcdCus : n_tiles <= 4 * kXcds * kXcdCus ? 16 : 4;
+inline int xcd_run(int n_tiles, int grid, int span) {
+  int run = 4;
+  if (n_tiles <= 4 * kXcds * kXcdCus) {
+    const int most = n_tiles <= kXcds * kXcdCus ? kXcdCus : 16;
+    while (2 * run * span <= kXcdCus && run < most) run *= 2;
+  }
   return run < grid / kXcds ? run : grid / kXcds;
 }
 // Launches with at most this many tiles (one workgroup per CU of an MI355X)
@@ -204,9 +215,10 @@ inline int step_variant(int n_tiles, double matrix_bytes, int tail_tiles = kTail
   if (n_tiles <= tail_tiles) return kStepTail;
   return matrix_bytes > stream_threshold() ? kStepStream : kStepCached;
 }
-// layout 0: runs of xcd_run tiles rotating over the XCDs; 1: per-QP chunks
-// (one contiguous chunk of every QP per XCD).  Results do not depend on it.
-void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int layout = 0);
+// Tiles of up to `span` slices.  layout 0: runs of xcd_run tiles rotating over
+// the XCDs; 1: per-QP chunks (one contiguous chunk of every QP per XCD).
+// Results do not depend on it.
+void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int span, int layout = 0);
 long solve_step_bound(const mprgp_params &p);
 size_t solve_bytes(const mprgp_qp *q, const mprgp_params &p);
 // the descriptor and initial state only (no device work; a mixed-form QP's

@@ -149,7 +149,7 @@ extern "C" int mprgp_qp_solve_noalloc(mprgp_qp *q, const mprgp_params *params, m
     }
   }
   MPRGP_HIP(launch_setup_rows(s, q->A->d_dinv, q->cn, q->cf, q->cs, q->n));
-  const int run = xcd_run(n_tiles, grid);  // layout_tiles' runs of tiles per XCD
+  const int run = xcd_run(n_tiles, grid, span);  // layout_tiles' runs of tiles per XCD
   StateWords sw;
   std::memcpy(&sw, &st, sizeof(sw));
   noalloc_tables<<<(grid + 255) / 256, 256, 0, s>>>(base, d, sw, q->st, q->part, q->A->n_slices, span, n_tiles,
