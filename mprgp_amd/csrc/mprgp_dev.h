@@ -62,6 +62,8 @@ enum Op : int {
                  // p' formed at the gather from z and p, p'.AP
   OP_CG_YA,      // FP64, after the first CG step: CG_Y without A x, then CG_A
                  // applied speculatively (beta into the other beta buffer)
+  OP_CG_PY,      // FP64, before CG_Y and CG_YA in the launch shapes whose
+                 // products gather P(y) instead of forming it: P(y) stored
   OP_NUM
 };
 

@@ -265,10 +265,36 @@ __device__ __forceinline__ void spmv_row(const int *sl_off, const C *col, const 
       acc);
 }
 
+// The one-vector SpMVs' unroll: the blocks of UB rows' slots are loaded per
+// round.  The sums still run over the blocks in order, so UB changes no bit
+// of a result.  kUnrollTail, with more registers and fewer waves, is for
+// launches with few tiles, where a lone row's chain of load rounds sets the
+// launch time.
+#ifndef MPRGP_STEP_UNROLL
+#define MPRGP_STEP_UNROLL 3
+#endif
+constexpr int kUnroll = MPRGP_STEP_UNROLL;
+constexpr int kUnrollTail = 6;
+
 // The projected gathers hold x, p and the row data of every block in flight:
 // two blocks where the one-vector SpMV takes three, four where it takes six,
 // keep the kernel without spills.
 constexpr int proj_unroll(int ub) { return ub > 3 ? 4 : 2; }
+
+// Whether a CG step's P(y) is formed by a launch of its own (CG_PY), which the
+// product then gathers, instead of at the gathers (spmv_proj: twice the
+// vector loads, and code the second slice of a wavefront repeats).  Where a
+// launch has at most a tile per CU and a tile is eight wavefronts, or a
+// wavefront two slices, the CU's loads and the instruction cache bound the
+// product, and the gathers cost more than the launch they save.  FP64 solves
+// of 1,984 and 7,139 nodes, own launch / at the gathers, us: tiles of 8
+// 2,453 / 2,699 and 2,822 / 2,924; two slices a wavefront 1,449 / 1,796 and
+// 1,792 / 2,219; both 3,841 / 4,924 and 4,793 / 5,873.  Smaller tiles stay at
+// the gathers: tiles of 4 1,623 / 1,706 and 1,859 / 1,849, tiles of 1 1,046 /
+// 1,025 and 1,275 / 1,255.  So do launches of more tiles, which their streams
+// bound (24 QPs, tiles of 8: 17.4 ms with own launches, 15.3 ms).  The results
+// are the same bits.
+constexpr bool split_trial(int ts, int spw, int ub) { return ub == kUnrollTail && (ts == 8 || spw == 2); }
 
 // A P(w) for w = x - alpha p (STEP) or w = x, with w and its projection
 // formed at the gather from the neighbours' x, p and rows, none of which the
@@ -549,7 +575,7 @@ __device__ __forceinline__ void next_outer_head(QpState &st, const Sums &S) {
 // Consumes the reduced partial sums of the op a QP executed in the previous
 // launch and moves its state machine to the next op (MPRGPSolver.h:42-79,
 // 148-456).  Every tile of the QP runs it on identical inputs.
-__device__ void control(QpState &st, const Sums &S) {
+__device__ void control(QpState &st, const Sums &S, bool split) {
   switch (st.op) {
     case OP_PROJX:
       st.op = st.pow_next;
@@ -602,7 +628,10 @@ __device__ void control(QpState &st, const Sums &S) {
       st.alpha = st.zg / st.pd;
       if (st.mixed && st.cg_entry) st.fx_entry = 0.5 * S.v[2];  // f(x) = x'(g - b)/2, g = A x - b
       // the CG entry needs f(x) too (four sums): its FP64 step takes CG_Y, CG_A
-      st.op = st.mixed ? OP_CG_PYG : OP_CG_Y;
+      st.op = st.mixed ? OP_CG_PYG : split ? OP_CG_PY : OP_CG_Y;
+      break;
+    case OP_CG_PY:
+      st.op = st.cg_entry ? OP_CG_Y : OP_CG_YA;
       break;
     case OP_CG_PYG: {
       // mixed inner solve: f(y) = f(x) - alpha p'g + alpha^2 p'Ap/2 and
@@ -648,7 +677,7 @@ __device__ void control(QpState &st, const Sums &S) {
       st.pb ^= 1;  // p' went to the other buffer
       st.pd = S.v[0];
       st.alpha = st.zg / st.pd;
-      st.op = st.mixed ? OP_CG_PYG : OP_CG_YA;
+      st.op = st.mixed ? OP_CG_PYG : split ? OP_CG_PY : OP_CG_YA;
       break;
     case OP_EXP2:
       st.xb ^= 1;  // the new x went to the other buffer
@@ -812,7 +841,7 @@ __device__ __forceinline__ auto cols(const QpDev &q) {
     return q.col;
 }
 
-template <class T, bool MX, int UB, bool NT, bool C16>
+template <class T, bool MX, int UB, bool NT, bool C16, bool SPLIT>
 __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int s, int lane, int r, int op,
                                          const QpState &st, double (&P)[kNumPart]) {
   const bool mixed = MX && st.mixed;
@@ -989,7 +1018,13 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       // the CG entry: y = x - alpha p, f(P(y)) and f(x)  (MPRGPSolver.h:276-284)
       if constexpr (std::is_same_v<T, double>) {
         V3 acc[2];
-        spmv_proj<2, UB / 3, NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
+        if constexpr (SPLIT)
+          spmv_row<2, 1, NT>(q.sl_off, cols<C16>(q), v.val, s, lane, [&](int j, V3 (&xs)[2]) {
+            xs[0] = ld3(v.py, j);
+            xs[1] = ld3(xc, j);
+          }, acc);
+        else
+          spmv_proj<2, UB / 3, NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
         const V3 xr = ld3(xc, r), pr = ld3(v.p, r);  // in flight with the row flag
         Row R = ldrow(q, v, r);
         const V3 y = axmy(xr, st.alpha, pr);
@@ -1003,6 +1038,14 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       }
       break;
     }
+    case OP_CG_PY: {  // P(y) of the trial point y = x - alpha p (split_trial)
+      if constexpr (std::is_same_v<T, double>) {
+        const V3 xr = ld3(xc, r), pr = ld3(v.p, r);  // in flight with the row flag
+        Row R = ldrow(q, v, r);
+        st3(v.py, r, proj(R, axmy(xr, st.alpha, pr)));
+      }
+      break;
+    }
     case OP_CG_YA: {
       // CGMonotonicStep (MPRGPSolver.h:281-302) after the CG entry: the trial
       // point y = x - alpha p and its feasibility, f(P(y)) by A P(y) with
@@ -1013,7 +1056,10 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       // the other buffer, current only once the step is accepted.
       if constexpr (!std::is_same_v<T, double>) break;
       V3 acc[1];
-      spmv_proj<1, proj_unroll(UB), NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
+      if constexpr (SPLIT)
+        spmv_row<1, UB, NT>(q.sl_off, cols<C16>(q), v.val, s, lane, [&](int j, V3 (&xs)[1]) { xs[0] = ld3(v.py, j); }, acc);
+      else
+        spmv_proj<1, proj_unroll(UB), NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
       const V3 xr = ld3(xc, r), pr = ld3(v.p, r);
       const bool f = gmem(q.face)[r];  // in flight with the row flag
       const V3 ap = ld3(v.ap, r), gr = ld3(v.g, r);
@@ -1263,17 +1309,18 @@ __device__ __forceinline__ bool fp64_op(int op) {
 }
 
 // One slice of a tile per wavefront.
-template <int TS, bool MX, int UB, bool NT, bool C16>
+template <int TS, bool MX, int UB, bool NT, int SPW, bool C16>
 __device__ __forceinline__ void slice_work(const QpDev &q, int s, int lane, int op, const QpState &st,
                                            double (&P)[kNumPart]) {
+  constexpr bool SPLIT = split_trial(TS, SPW, UB);
   const int r = s * kSlice + lane;
   if (r >= q.n_nodes) return;
   if (fp64_op(op)) {
     row_work_fp64<MX, UB, NT, C16>(q, s, lane, r, op, st, P);
   } else if (MX && st.mixed) {
-    row_work<float, MX, UB, NT, C16>(q, q.f, s, lane, r, op, st, P);
+    row_work<float, MX, UB, NT, C16, SPLIT>(q, q.f, s, lane, r, op, st, P);
   } else {
-    row_work<double, MX, UB, NT, C16>(q, q.d, s, lane, r, op, st, P);
+    row_work<double, MX, UB, NT, C16, SPLIT>(q, q.d, s, lane, r, op, st, P);
   }
 }
 
@@ -1288,11 +1335,11 @@ __device__ void tile_work(const QpDev &q, const Tile &t, int op, const QpState &
   const int wave = threadIdx.x / kSlice;
   const int lane = threadIdx.x % kSlice;
   if constexpr (SPW == 1) {
-    if (wave < t.slices) slice_work<TS, MX, UB, NT, C16>(q, t.slice0 + wave, lane, op, st, P);
+    if (wave < t.slices) slice_work<TS, MX, UB, NT, SPW, C16>(q, t.slice0 + wave, lane, op, st, P);
   } else {
     static_assert(SPW == 2, "one or two slices per wavefront");
-    if (wave < t.slices) slice_work<TS, MX, UB, NT, C16>(q, t.slice0 + wave, lane, op, st, P);
-    if (wave + TS < t.slices) slice_work<TS, MX, UB, NT, C16>(q, t.slice0 + wave + TS, lane, op, st, P);
+    if (wave < t.slices) slice_work<TS, MX, UB, NT, SPW, C16>(q, t.slice0 + wave, lane, op, st, P);
+    if (wave + TS < t.slices) slice_work<TS, MX, UB, NT, SPW, C16>(q, t.slice0 + wave + TS, lane, op, st, P);
   }
 }
 
@@ -1369,17 +1416,6 @@ typedef uint64_t __attribute__((__may_alias__)) StateWord;
 #define MPRGP_STEP_MIN_WAVES 4
 #endif
 
-// The one-vector SpMVs' unroll: the blocks of UB rows' slots are loaded per
-// round.  The sums still run over the blocks in order, so UB changes no bit
-// of a result.  kUnrollTail, with more registers and fewer waves, is for
-// launches with few tiles, where a lone row's chain of load rounds sets the
-// launch time.
-#ifndef MPRGP_STEP_UNROLL
-#define MPRGP_STEP_UNROLL 3
-#endif
-constexpr int kUnroll = MPRGP_STEP_UNROLL;
-constexpr int kUnrollTail = 6;
-
 // MX: the batch holds QPs of the mixed form (their inner ops run on the FP32
 // copies); FP64 QPs of the same batch take the FP64 path.  C16: every QP of
 // the batch has 16-bit column indices (QpDev::col16).
@@ -1433,7 +1469,7 @@ __global__ void __launch_bounds__(TS * kSlice, UB == kUnroll ? MPRGP_STEP_MIN_WA
     if (lane == 0) {
       const bool skip = sst.fresh || sst.op == OP_DONE;
       const bool was_done = sst.op == OP_DONE;
-      if (!skip) control(sst, S);
+      if (!skip) control(sst, S, split_trial(TS, SPW, UB));
       sst.fresh = 0;
       if (t.local == 0) {  // the QP's first tile counts the launch (or its end)
         if (sst.op != OP_DONE) {

@@ -17,7 +17,7 @@ from mprgp_amd import problems
 OPS = ["DONE", "PROJX", "POW_IT", "POW_SAVE", "INIT", "TOP", "CG_AP", "CG_Y",
        "CG_A", "EXP2", "EXP3", "PROP1", "PROP2", "FINAL", "CL_AP", "CL_CG",
        "CL_EXP", "CL_EXP2", "CL_PROP1", "R_START", "R_UPD", "R_FINAL", "CG_PYG",
-       "CG_BAP", "CG_YA"]
+       "CG_BAP", "CG_YA", "CG_PY"]
 
 
 class DeviceQP:
@@ -59,6 +59,7 @@ _STREAMS = {
     "CG_A": ("rows", "face", "ap", "g", "dinv", "x", "g", "phi", "z", "beta"),
     "CG_PYG": ("rows", "face", "x", "p", "y", "g", "ap", "dinv", "g", "phi", "z", "beta"),
     "CG_BAP": ("M", "z", "p", "p", "ap"),
+    "CG_PY": ("rows", "x", "p", "py"),
     "CG_YA": ("M", "x", "p", "y", "b", "rows", "face", "ap", "g", "dinv", "g", "phi", "z", "beta"),
     "EXP2": ("M", "x", "b", "rows", "py", "x"),
     "PROP1": ("M", "x", "beta", "b", "g", "ap"),
