@@ -107,7 +107,8 @@ typedef struct {
   int ev_valid;       /* power vector stored for the next solve                     */
   int refinements;    /* MIXED: outer refinement sweeps                             */
   int steps;          /* device launches this QP took part in                       */
-  int launches;       /* step-kernel launches issued for the whole call             */
+  int launches;       /* step-kernel launches issued for the whole call; coupled    */
+                      /* solve: launches of its one-workgroup loop (0: from host)   */
   int fp64_finish;    /* MIXED: 1 when every refinement sweep ran and the residual  */
                       /* was still above tol (the FP32 inner solve's floor), so the */
                       /* FP64 form finished the solve from that x; then iterations  */

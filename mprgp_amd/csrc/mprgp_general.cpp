@@ -274,6 +274,7 @@ struct General {
   // The one-workgroup loop (mprgp_general_dev.hip) takes the main loop: its
   // components, packed, and its share of the device block.
   bool one_launch = false;
+  int loop_launches = 0;
   std::vector<int> big_row, one_row;
   std::vector<double> big_g, one_g;
   GenArgs *d_args = nullptr;
@@ -281,9 +282,15 @@ struct General {
   double *d_c = nullptr, *d_big_g = nullptr, *d_one_g = nullptr;
   int *d_big_row = nullptr, *d_one_row = nullptr;
   unsigned char *d_face = nullptr;
-  void pack_components(int n_nodes) {
+  void pack_components(int n_nodes, long long slots) {
     one_launch = m > 0 && m <= kGenMaxRows && n_nodes <= kGenMaxNodes;
-    for (const auto &rows : comps) one_launch = one_launch && rows.size() <= (size_t)kGenBlock;
+    double gain = kGenGain - kGenNodeCost * n_nodes - kGenSlotCost * slots;
+    for (const auto &rows : comps) {
+      const int k = (int)rows.size();
+      one_launch = one_launch && k <= kGenBlock;
+      gain += k == 1 ? kGenRowGain : -(kGenCompCost1 * k + kGenCompCost2 * k * k);
+    }
+    one_launch = one_launch && gain > 0.0;
     if (!one_launch) return;
     for (size_t c0 = 0; c0 < comps.size(); ++c0) {
       const int k = (int)comps[c0].size();
@@ -313,6 +320,7 @@ struct General {
     MPRGP_HIP(hipStreamSynchronize(s));  // a is a local
     while (!st->done && !st->fail) {
       MPRGP_HIP(launch_general_loop(s, d_args));
+      ++loop_launches;
       MPRGP_HIP(hipMemcpyAsync(h_rb, d_state, sizeof(*st), hipMemcpyDeviceToHost, s));
       MPRGP_HIP(hipStreamSynchronize(s));
       std::memcpy(st, h_rb, sizeof(*st));
@@ -686,7 +694,7 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
   G.c.assign(c, c + m);
   if (int rc = G.build_jjt(j_ptr, j_val, jc, tptr, tc)) return rc;
   G.face.assign(m, 0);
-  G.pack_components(q->n);
+  G.pack_components(q->n, q->A->slots);
   // device block: J, J^T, J v, lambda, dot partials and results
   const size_t parts = ((size_t)n + 255) / 256 + 1;
   const size_t bytes = sizeof(int) * ((size_t)m + 1 + (size_t)nnz + (size_t)n + 1 + (size_t)nnz) +
@@ -943,6 +951,7 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
     stats->active = (int)G.act.size();
     stats->power_iters = piters;
     stats->ev_valid = q->ev_valid;
+    stats->launches = G.loop_launches;
     stats->residual = residual;
     stats->alpha_bar = alpha_bar;
     stats->lambda_max = lmax;

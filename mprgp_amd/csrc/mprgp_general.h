@@ -15,6 +15,21 @@ constexpr int kGenBlock = 6;
 // nodes, but its products with A, on one CU, grow with the matrix.
 constexpr int kGenMaxNodes = 2600;
 constexpr int kGenMaxRows = 16384;  // some two rows per entry of the largest vector
+// What the one-workgroup loop gains on the host-driven one, microseconds an
+// iteration: the launches and waits it saves, and about 0.07 for a row that
+// shares nodes with no other (three QPs on the host); less the time one CU
+// takes for the vectors, the matrix (its load path) and the components of
+// several rows (a wavefront each, 16 at a time; the host factors a block in
+// less than a wavefront does).  The loop is taken where the estimate is
+// positive.  Fitted low to 360 pairs of both loops' times (100 to 2,600 nodes, 3 to
+// 300 blocks a row, 0 to 512 components of 1 to 6 rows, none to all of their
+// rows active, CG and expansion steps), so that none of those estimated
+// positive was slower than from the host: 2,600 nodes, host / one workgroup:
+// 3 blocks a row, 8 pairs of rows 202 / 95 us, 256 pairs 313 / 339, 512
+// components of six 800 / 1,473; 27 blocks a row, 8 pairs 210 / 242.  A beam
+// of 525 nodes with 525 ground rows and 12 contacts 344 / 105.
+constexpr double kGenGain = 145.0, kGenRowGain = 0.07, kGenNodeCost = 0.03, kGenSlotCost = 0.0019;
+constexpr double kGenCompCost1 = 0.1, kGenCompCost2 = 0.0175;  // k rows: 0.1 k + 0.0175 k^2
 // Iterations per launch, so that no launch runs long.
 constexpr int kGenChunk = 256;
 
