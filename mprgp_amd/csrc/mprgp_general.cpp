@@ -695,15 +695,18 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
   if (int rc = G.build_jjt(j_ptr, j_val, jc, tptr, tc)) return rc;
   G.face.assign(m, 0);
   G.pack_components(q->n, q->A->slots);
-  // device block: J, J^T, J v, lambda, dot partials and results
+  // device block: J, J^T, J v, lambda, dot partials and results, and what the
+  // one-workgroup loop adds; where that is refused, the host drives the loop
   const size_t parts = ((size_t)n + 255) / 256 + 1;
   const size_t bytes = sizeof(int) * ((size_t)m + 1 + (size_t)nnz + (size_t)n + 1 + (size_t)nnz) +
-                       sizeof(double) * (2 * (size_t)nnz + 5 * ((size_t)m + 1) + kMaxDots * parts + 16) + 1024 +
-                       (G.one_launch ? sizeof(GenArgs) + sizeof(GenState) + sizeof(double) * (G.big_g.size() + 2 * (size_t)m) +
-                                           sizeof(int) * (G.big_row.size() + (size_t)m) + (size_t)m
-                                     : 0);
-  if (int rc = ctx->alloc(&G.blk, bytes)) return rc;
-  G.blk_bytes = bytes;
+                       sizeof(double) * (2 * (size_t)nnz + 5 * ((size_t)m + 1) + kMaxDots * parts + 16) + 1024;
+  G.blk_bytes = bytes + sizeof(GenArgs) + sizeof(GenState) + sizeof(double) * (G.big_g.size() + 2 * (size_t)m) +
+                sizeof(int) * (G.big_row.size() + (size_t)m) + (size_t)m;
+  G.one_launch = G.one_launch && ctx->alloc(&G.blk, G.blk_bytes) == MPRGP_OK;
+  if (!G.one_launch) {
+    if (int rc = ctx->alloc(&G.blk, bytes)) return rc;
+    G.blk_bytes = bytes;
+  }
   if (hipHostMalloc((void **)&G.h_lam, sizeof(double) * (5 * ((size_t)m + 1) + 16), hipHostMallocDefault) !=
       hipSuccess) {
     G.h_lam = nullptr;

@@ -68,3 +68,23 @@ def test_ica_without_room_for_the_ring(ctx):
     with pytest.raises(M.MprgpError) as e:
         on_budget(A, b, x0, call, least - 2048)
     assert e.value.code == -7
+
+
+def test_coupled_solve_without_room_for_the_one_workgroup_loop(ctx):
+    A, b, J, c, x0 = beam()
+    n, m, nnz = A.shape[0], J.shape[0], J.nnz
+    parts = (n + 255) // 256 + 1
+    least = 4 * (m + 1 + nnz + n + 1 + nnz) + 8 * (2 * nnz + 5 * (m + 1) + 8 * parts + 16) + 1024
+
+    def call(q):
+        rc, st = M.general_solve(q, J, c, tol=1e-9, max_it=60, alpha_bar=1e-3, project_first=1)
+        return [rc] + [st[f] for f in ("iterations", "num_cg", "num_exp", "num_prop", "active", "residual")], \
+            st["launches"]
+    (free, loop), xf = on_budget(A, b, x0, call)
+    (tight, host), xt = on_budget(A, b, x0, call, least)
+    assert loop > 0 and host == 0
+    assert tight == free
+    np.testing.assert_array_equal(xt, xf)
+    with pytest.raises(M.MprgpError) as e:
+        on_budget(A, b, x0, call, least - 1)
+    assert e.value.code == -7
