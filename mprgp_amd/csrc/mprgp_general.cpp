@@ -277,11 +277,19 @@ struct General {
   int loop_launches = 0;
   std::vector<int> big_row, one_row;
   std::vector<double> big_g, one_g;
-  GenArgs *d_args = nullptr;
-  GenState *d_state = nullptr;
+  // Device: one block that goes up and comes back in one copy, pinned on the
+  // host (a solve that meets its tolerance at once lasts no longer than its
+  // copies): the arguments, the state and the face.  And what a solve only
+  // reads: c, the components' blocks of J J^T and rows.
+  struct Control {
+    GenArgs args;
+    GenState st;
+    unsigned char face[];
+  };
+  Control *d_ctl = nullptr, *h_ctl = nullptr;
+  size_t ctl_bytes() const { return sizeof(Control) + (size_t)m; }
   double *d_c = nullptr, *d_big_g = nullptr, *d_one_g = nullptr;
   int *d_big_row = nullptr, *d_one_row = nullptr;
-  unsigned char *d_face = nullptr;
   void pack_components(int n_nodes, long long slots) {
     one_launch = m > 0 && m <= kGenMaxRows && n_nodes <= kGenMaxNodes;
     double gain = kGenGain - kGenNodeCost * n_nodes - kGenSlotCost * slots;
@@ -310,24 +318,21 @@ struct General {
   int loop_on_device(double alpha_bar, double tol, int max_it, bool pre, GenState *st) {
     const mprgp_matrix *A = q->A;
     const GenArgs a{n, m, A->n_nodes, A->n_slices, A->d_sl_off, A->d_col, A->d_val, dinv, b, x, g, p, z, phi, beta,
-                    y, gp, t, t2, t3, tl, jp, jc, tp, tc, jv, tv, d_c, d_face, jslot(0), jslot(1), lam, lam + m + 1, part,
+                    y, gp, t, t2, t3, tl, jp, jc, tp, tc, jv, tv, d_c, d_ctl->face, jslot(0), jslot(1), lam, lam + m + 1, part,
                     (int)big_row.size() / kGenBlock, (int)one_row.size(), d_big_row, d_one_row, d_big_g, d_one_g,
-                    alpha_bar, tol, max_it, pre, kGenChunk, d_state};
-    *st = GenState{};
-    MPRGP_HIP(hipMemcpyAsync(d_args, &a, sizeof(a), hipMemcpyHostToDevice, s));
-    MPRGP_HIP(hipMemcpyAsync(d_state, st, sizeof(*st), hipMemcpyHostToDevice, s));
-    MPRGP_HIP(hipMemcpyAsync(d_face, face.data(), (size_t)m, hipMemcpyHostToDevice, s));
-    MPRGP_HIP(hipStreamSynchronize(s));  // a is a local
-    while (!st->done && !st->fail) {
-      MPRGP_HIP(launch_general_loop(s, d_args));
+                    alpha_bar, tol, max_it, pre, kGenChunk, &d_ctl->st};
+    h_ctl->args = a;
+    h_ctl->st = GenState{};
+    std::copy(face.begin(), face.end(), h_ctl->face);
+    MPRGP_HIP(hipMemcpyAsync(d_ctl, h_ctl, ctl_bytes(), hipMemcpyHostToDevice, s));
+    do {
+      MPRGP_HIP(launch_general_loop(s, &d_ctl->args));
       ++loop_launches;
-      MPRGP_HIP(hipMemcpyAsync(h_rb, d_state, sizeof(*st), hipMemcpyDeviceToHost, s));
+      MPRGP_HIP(hipMemcpyAsync(&h_ctl->st, &d_ctl->st, ctl_bytes() - offsetof(Control, st), hipMemcpyDeviceToHost, s));
       MPRGP_HIP(hipStreamSynchronize(s));
-      std::memcpy(st, h_rb, sizeof(*st));
-    }
-    MPRGP_HIP(hipMemcpyAsync(h_rb, d_face, (size_t)m, hipMemcpyDeviceToHost, s));
-    MPRGP_HIP(hipStreamSynchronize(s));
-    std::memcpy(face.data(), h_rb, (size_t)m);
+    } while (!h_ctl->st.done && !h_ctl->st.fail);
+    *st = h_ctl->st;
+    std::copy(h_ctl->face, h_ctl->face + m, face.begin());
     act.clear();
     for (int i = 0; i < m; ++i)
       if (face[i]) act.push_back(i);
@@ -694,25 +699,28 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
   G.c.assign(c, c + m);
   if (int rc = G.build_jjt(j_ptr, j_val, jc, tptr, tc)) return rc;
   G.face.assign(m, 0);
-  G.pack_components(q->n, q->A->slots);
+  if (p.max_it > 0) G.pack_components(q->n, q->A->slots);
   // device block: J, J^T, J v, lambda, dot partials and results, and what the
   // one-workgroup loop adds; where that is refused, the host drives the loop
   const size_t parts = ((size_t)n + 255) / 256 + 1;
   const size_t bytes = sizeof(int) * ((size_t)m + 1 + (size_t)nnz + (size_t)n + 1 + (size_t)nnz) +
                        sizeof(double) * (2 * (size_t)nnz + 5 * ((size_t)m + 1) + kMaxDots * parts + 16) + 1024;
-  G.blk_bytes = bytes + sizeof(GenArgs) + sizeof(GenState) + sizeof(double) * (G.big_g.size() + 2 * (size_t)m) +
-                sizeof(int) * (G.big_row.size() + (size_t)m) + (size_t)m;
+  const size_t read_bytes = sizeof(double) * ((size_t)m + G.big_g.size() + G.one_g.size()) +
+                            sizeof(int) * (G.big_row.size() + G.one_row.size());
+  G.blk_bytes = bytes + G.ctl_bytes() + read_bytes;
   G.one_launch = G.one_launch && ctx->alloc(&G.blk, G.blk_bytes) == MPRGP_OK;
   if (!G.one_launch) {
     if (int rc = ctx->alloc(&G.blk, bytes)) return rc;
     G.blk_bytes = bytes;
   }
-  if (hipHostMalloc((void **)&G.h_lam, sizeof(double) * (5 * ((size_t)m + 1) + 16), hipHostMallocDefault) !=
+  const size_t lam_bytes = sizeof(double) * (5 * ((size_t)m + 1) + 16);
+  if (hipHostMalloc((void **)&G.h_lam, lam_bytes + (G.one_launch ? G.ctl_bytes() : 0), hipHostMallocDefault) !=
       hipSuccess) {
     G.h_lam = nullptr;
     return fail(MPRGP_ENOMEM, "pinned staging of %d multipliers", m);
   }
   G.h_rb = G.h_lam + 2 * ((size_t)m + 1);
+  G.h_ctl = (General::Control *)((char *)G.h_lam + lam_bytes);
   {
     char *b8 = (char *)G.blk;
     auto carve = [&](size_t sz) {
@@ -731,14 +739,12 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
     G.tp = (int *)carve(sizeof(int) * (n + 1));
     G.tc = (int *)carve(sizeof(int) * nnz);
     if (G.one_launch) {
-      G.d_args = (GenArgs *)carve(sizeof(GenArgs));
-      G.d_state = (GenState *)carve(sizeof(GenState));
-      G.d_c = (double *)carve(sizeof(double) * m);
-      G.d_big_g = (double *)carve(sizeof(double) * G.big_g.size());
-      G.d_one_g = (double *)carve(sizeof(double) * G.one_g.size());
-      G.d_big_row = (int *)carve(sizeof(int) * G.big_row.size());
-      G.d_one_row = (int *)carve(sizeof(int) * G.one_row.size());
-      G.d_face = (unsigned char *)carve(m);
+      G.d_c = (double *)carve(read_bytes);
+      G.d_big_g = G.d_c + m;
+      G.d_one_g = G.d_big_g + G.big_g.size();
+      G.d_big_row = (int *)(G.d_one_g + G.one_g.size());
+      G.d_one_row = G.d_big_row + G.big_row.size();
+      G.d_ctl = (General::Control *)carve(G.ctl_bytes());
     }
   }
   hipStream_t s = G.s;
@@ -750,16 +756,16 @@ extern "C" int mprgp_general_solve(mprgp_qp *q, int m, const int *j_ptr, const i
     MPRGP_HIP(hipMemcpyAsync(G.tv, tv.data(), sizeof(double) * nnz, hipMemcpyHostToDevice, s));
   }
   MPRGP_HIP(hipMemcpyAsync(G.tp, tptr.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, s));
+  std::vector<char> read;  // as it lies on the device
   if (G.one_launch) {
-    MPRGP_HIP(hipMemcpyAsync(G.d_c, c, sizeof(double) * m, hipMemcpyHostToDevice, s));
-    if (!G.big_row.empty()) {
-      MPRGP_HIP(hipMemcpyAsync(G.d_big_g, G.big_g.data(), sizeof(double) * G.big_g.size(), hipMemcpyHostToDevice, s));
-      MPRGP_HIP(hipMemcpyAsync(G.d_big_row, G.big_row.data(), sizeof(int) * G.big_row.size(), hipMemcpyHostToDevice, s));
-    }
-    if (!G.one_row.empty()) {
-      MPRGP_HIP(hipMemcpyAsync(G.d_one_g, G.one_g.data(), sizeof(double) * G.one_g.size(), hipMemcpyHostToDevice, s));
-      MPRGP_HIP(hipMemcpyAsync(G.d_one_row, G.one_row.data(), sizeof(int) * G.one_row.size(), hipMemcpyHostToDevice, s));
-    }
+    read.reserve(read_bytes);
+    auto put = [&](const auto *v, size_t k) { read.insert(read.end(), (const char *)v, (const char *)(v + k)); };
+    put(c, m);
+    put(G.big_g.data(), G.big_g.size());
+    put(G.one_g.data(), G.one_g.size());
+    put(G.big_row.data(), G.big_row.size());
+    put(G.one_row.data(), G.one_row.size());
+    MPRGP_HIP(hipMemcpyAsync(G.d_c, read.data(), read_bytes, hipMemcpyHostToDevice, s));
   }
   MPRGP_HIP(hipStreamSynchronize(s));  // the host arrays above are locals
   G.x = q->x; G.g = q->g; G.p = q->p; G.z = q->z; G.phi = q->phi; G.beta = q->beta; G.y = q->y;

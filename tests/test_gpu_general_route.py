@@ -53,3 +53,11 @@ def test_matrix_decides(ctx, n, band, one):
     J[0, 0:6], J[1, 3:6] = rng.standard_normal(6), rng.standard_normal(3)
     st, _ = solve(ctx, A, 0.05 * rng.standard_normal(3 * n), J.tocsr(), np.array([-0.1, 0.1]), max_it=10)
     assert (st["launches"] > 0) == one
+
+
+def test_without_iterations_no_loop_is_launched(ctx):
+    rng = np.random.default_rng(1)
+    A, b = chain(rng, 300)
+    J, c = rows_on(rng, 300, 5, 12)
+    st, _ = solve(ctx, A, b, J, c, max_it=0)
+    assert st["launches"] == 0 and st["iterations"] == 0
