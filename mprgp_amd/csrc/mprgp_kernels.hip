@@ -239,6 +239,7 @@ __device__ __forceinline__ void spmv_round(CP cp, VP vp, int k, int n, G &gather
 template <int NV, int U, bool NT, class C, class T, class G>
 __device__ __forceinline__ void spmv_rounds(const int *sl_off, const C *col, const T *val, int s, int lane,
                                             G gather_all, V3 (&acc)[NV]) {
+  static_assert(U >= 1, "a round of no blocks would never end");
 #pragma unroll
   for (int t = 0; t < NV; ++t) acc[t] = V3{0.0, 0.0, 0.0};
   const int b0 = gmem(sl_off)[s];
@@ -280,6 +281,8 @@ constexpr int kUnrollTail = 6;
 // two blocks where the one-vector SpMV takes three, four where it takes six,
 // keep the kernel without spills.
 constexpr int proj_unroll(int ub) { return ub > 3 ? 4 : 2; }
+// Blocks in flight where x and P(y) are gathered together.
+constexpr int pair_unroll(int ub) { return ub >= 3 ? ub / 3 : 1; }
 
 // Whether a CG step's P(y) is formed by a launch of its own (CG_PY), which the
 // product then gathers, instead of at the gathers (spmv_proj: twice the
@@ -1024,7 +1027,7 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
             xs[1] = ld3(xc, j);
           }, acc);
         else
-          spmv_proj<2, UB / 3, NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
+          spmv_proj<2, pair_unroll(UB), NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
         const V3 xr = ld3(xc, r), pr = ld3(v.p, r);  // in flight with the row flag
         Row R = ldrow(q, v, r);
         const V3 y = axmy(xr, st.alpha, pr);
