@@ -17,7 +17,8 @@
 // are grouped into dependency levels (a node's level is one more than the
 // highest level among the nodes it couples to that come before it), and one
 // workgroup runs the levels in order with a barrier between them, x in an
-// LDS ring where the levels' reach allows (ica_sweep_ring).  Every node then sees exactly the new and old values the sequential sweep gives
+// LDS ring where the levels' reach allows (ica_sweep_ring).  Every node then
+// sees exactly the new and old values the sequential sweep gives
 // it, so the sweep is the reference's, not a multicolour variant with other
 // iterates.  Each row adds its terms in the order of its blocks (the input's
 // column order), singly rounded, as the oracle does.
@@ -221,13 +222,18 @@ constexpr int kSweepThreads = 512;
 //   lo_cnt    per position: the node's lower blocks
 //   dinv, rhs per position; node: the internal node at a position
 // Used where every column a level reads is among the kRing positions up to
-// the level's end (the caller checks); a level past 256 nodes runs in passes.
+// the level's end (the caller checks); a level past 128 nodes (four lanes each)
+// runs in passes.
 // Measured on a beam of 3,402 nodes in 148 levels: an iteration 443 -> 222 us
 // (with the wait merged below); what is left per level is the load path of
 // one CU, about 35 bytes a cycle.
 constexpr int kRing = 6400;  // 150 KB of x; the 44,541-node beam's levels read at most 881 positions back
 constexpr int kAhead = 9;    // a node of the beams has at most 9 lower blocks
 constexpr int kRingThreads = 512;
+// A level of more nodes than the ring has slots (one without lower blocks)
+// writes a slot in several passes with no barrier between them: the last one
+// stands because the same quad writes them all, in order.
+static_assert(kRing % (kRingThreads / 4) == 0, "a ring slot belongs to one quad of the workgroup");
 struct SweepLevel {
   int t0, count, base, blocks;
 };
