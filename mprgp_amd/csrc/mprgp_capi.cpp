@@ -1238,8 +1238,40 @@ extern "C" int mprgp_qp_get_rows(mprgp_qp *q, int cap, int *m, int *node, double
 
 namespace mprgp {
 
+namespace {
+// live drivers per XCD of each device; never freed, a context may outlive it
+std::mutex &start_mu() {
+  static std::mutex *m = new std::mutex();
+  return *m;
+}
+std::map<int, std::vector<int>> &start_use() {
+  static auto *u = new std::map<int, std::vector<int>>();
+  return *u;
+}
+}  // namespace
+void XcdStart::take(int device) {
+  give();
+  std::lock_guard<std::mutex> lock(start_mu());
+  std::vector<int> &use = start_use()[device];
+  use.resize(kXcds, 0);
+  int best = 0;
+  for (int x : {4, 2, 6, 1, 5, 3, 7})
+    if (use[x] < use[best]) best = x;
+  ++use[best];
+  xcd_ = best;
+  device_ = device;
+}
+void XcdStart::give() {
+  if (device_ < 0) return;
+  std::lock_guard<std::mutex> lock(start_mu());
+  --start_use()[device_][xcd_];
+  device_ = -1;
+  xcd_ = 0;
+}
+
 int BatchTables::init(mprgp_ctx *ctx) {
   this->ctx = ctx;
+  start.take(ctx->device);
   if (int rc = ctx->alloc((void **)&d_ctrl, 4 * sizeof(int))) return rc;
   return MPRGP_OK;
 }
@@ -1253,6 +1285,7 @@ void BatchTables::drop_graphs() {
 
 void BatchTables::destroy() {
   if (!ctx) return;
+  start.give();
   drop_graphs();
   ctx->release(d_qps, sizeof(QpDev) * (size_t)qps_cap);
   ctx->release(d_tiles, sizeof(Tile) * (size_t)tiles_cap);
@@ -1459,7 +1492,7 @@ static bool layout_chunks(const std::vector<Tile> &tiles, int grid, Tile *table)
   return true;
 }
 
-void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int span, int layout) {
+void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int span, int xcd0, int layout) {
   if (layout == 1 && layout_chunks(tiles, grid, table)) return;
   const int n = (int)tiles.size();
   // grid and the run are powers of two, grid at least 64, so c * kXcds divides
@@ -1467,7 +1500,7 @@ void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int spa
   const int c = xcd_run(n, grid, span);
   for (int b = 0; b < grid; ++b) table[b] = Tile{nullptr, nullptr, -1, 0, 0, 0, 0, 0};
   for (int i = 0; i < n; ++i) {
-    const int xcd = (i / c) % kXcds, pos = (i / (c * kXcds)) * c + i % c;
+    const int xcd = (i / c + xcd0) % kXcds, pos = (i / (c * kXcds)) * c + i % c;
     table[pos * kXcds + xcd] = tiles[i];
   }
 }
@@ -1677,7 +1710,7 @@ static int run_batch(mprgp_ctx *ctx, int count, mprgp_qp *const *qps, const mprg
   if (int rc = tab.ensure(count, grid)) return rc;
   if (int rc = tab.ensure_states(count)) return rc;
   const int layout = params[0].xcd_layout;
-  layout_tiles(tiles, grid, tab.h_tiles, span, layout);
+  layout_tiles(tiles, grid, tab.h_tiles, span, tab.start.xcd(), layout);
   hipStream_t s = ctx->stream;
   std::vector<QpDev> devs(count);
   QpState *states = tab.h_states;  // pinned; [i][2]
@@ -1780,7 +1813,7 @@ static int run_batch(mprgp_ctx *ctx, int count, mprgp_qp *const *qps, const mprg
         for (int i = 0; i < count; ++i)
           if (keep[i]) append_tiles(i, qps[i], span, kept);
         grid = round_grid((int)kept.size());  // <= the table's capacity: the tile count only shrinks
-        layout_tiles(kept, grid, tab.h_tiles, span, layout);
+        layout_tiles(kept, grid, tab.h_tiles, span, tab.start.xcd(), layout);
         MPRGP_HIP(hipMemcpyAsync(tab.d_tiles, tab.h_tiles, sizeof(Tile) * grid, hipMemcpyHostToDevice, s));
         in_table = live;
         shrunk_at = k;

@@ -205,7 +205,7 @@ int mprgp_engine::round_once(long r, bool &idle) {
     tv.reserve(n_tiles);
     for (int i = 0; i < (int)slots.size(); ++i)
       if (slots[i].req && slots[i].retiring == 0) append_tiles(i, slots[i].req->q, ts, tv);
-    layout_tiles(tv, grid, tl, ts);
+    layout_tiles(tv, grid, tl, ts, tab.start.xcd());
     std::memcpy(h_qps[par].p, devs.data(), sizeof(QpDev) * devs.size());
     MPRGP_HIP(hipMemcpyAsync(tab.d_qps, h_qps[par].p, sizeof(QpDev) * devs.size(), hipMemcpyHostToDevice, s));
     MPRGP_HIP(hipMemcpyAsync(tab.d_tiles, tl, sizeof(Tile) * grid, hipMemcpyHostToDevice, s));

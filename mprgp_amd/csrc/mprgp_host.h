@@ -124,10 +124,35 @@ hipError_t launch_copy_stream(hipStream_t s, const void *in, void *out, size_t b
 int build_matrix(mprgp_ctx *ctx, int n_nodes, const int *rowptr, const int *colidx,
                  const double *blocks, mprgp_matrix **out);
 
+constexpr int kXcds = 8, kXcdCus = 32;
+
+// The XCD that the first tiles of a driver's launches stand on: of the
+// device's, one that the fewest live drivers have, halves apart first.  A
+// launch of few tiles stands on few XCDs (xcd_run), and drivers whose solves
+// run at the same time would share those while others idle.  Two contexts
+// solving 7,139 nodes (112 tiles, four XCDs) with the power method: 12.1 ms a
+// solve on the same four, 10.0 apart, 11.1 in runs of 4 over all eight; 4,100
+// nodes 10.3, 8.6 and 10.4; three contexts, which have to overlap, 12.8, 12.4
+// and 12.2.  31 tiles share an XCD without loss (7.9 ms either way).
+class XcdStart {
+ public:
+  XcdStart() = default;
+  XcdStart(const XcdStart &) = delete;
+  XcdStart &operator=(const XcdStart &) = delete;
+  ~XcdStart() { give(); }
+  void take(int device);
+  void give();
+  int xcd() const { return xcd_; }
+
+ private:
+  int device_ = -1, xcd_ = 0;
+};
+
 // Device launch tables of one batch driver (a context's solve_batch, or an
 // engine): QP descriptors, tiles, control words, done flags, captured graphs.
 struct BatchTables {
   mprgp_ctx *ctx = nullptr;
+  XcdStart start;
   QpDev *d_qps = nullptr;
   int qps_cap = 0;
   Tile *d_tiles = nullptr;  // one slot per workgroup of a launch (layout_tiles)
@@ -188,7 +213,6 @@ int round_grid(int n_tiles);
 //   and one XCD's share sets the launch time (256 QPs: runs of 4 0.7% faster
 //   than single tiles, runs of 16 1% slower, whole QPs per XCD 6% slower).
 // At least 4, and what the launch's slots hold.
-constexpr int kXcds = 8, kXcdCus = 32;
 inline int xcd_run(int n_tiles, int grid, int span) {
   int run = 4;
   if (n_tiles <= 4 * kXcds * kXcdCus) {
@@ -216,9 +240,9 @@ inline int step_variant(int n_tiles, double matrix_bytes, int tail_tiles = kTail
   return matrix_bytes > stream_threshold() ? kStepStream : kStepCached;
 }
 // Tiles of up to `span` slices.  layout 0: runs of xcd_run tiles rotating over
-// the XCDs; 1: per-QP chunks (one contiguous chunk of every QP per XCD).
-// Results do not depend on it.
-void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int span, int layout = 0);
+// the XCDs from xcd0; 1: per-QP chunks (one contiguous chunk of every QP per
+// XCD).  Results do not depend on it.
+void layout_tiles(const std::vector<Tile> &tiles, int grid, Tile *table, int span, int xcd0, int layout = 0);
 long solve_step_bound(const mprgp_params &p);
 size_t solve_bytes(const mprgp_qp *q, const mprgp_params &p);
 // the descriptor and initial state only (no device work; a mixed-form QP's

@@ -62,7 +62,7 @@ int noalloc_setup(int device) {
 // Writes the launch tables of one QP into the scratch array and both of the
 // QP's state copies: the descriptor, the running count (1), a cleared done
 // flag, and the tile table in layout_tiles' XCD order (slot b holds tile
-// i = (b/8/c)*8c + (b%8)*c + (b/8)%c, the inverse of its map, or nothing).
+// i = (b/8/c)*8c + ((b-xcd0)%8)*c + (b/8)%c, the inverse of its map, or nothing).
 // One thread per table slot; thread 0 of block 0 also writes the rest.
 struct StateWords {  // a QpState as a kernel argument (plain 8-byte words)
   uint64_t w[64];
@@ -71,11 +71,11 @@ static_assert(sizeof(QpState) == sizeof(StateWords), "a state copy is 64 words")
 
 __global__ void __launch_bounds__(256) noalloc_tables(unsigned char *base, QpDev d, StateWords st, QpState *qst,
                                                       double *part, int n_slices, int span, int n_tiles,
-                                                      int grid, int run) {
+                                                      int grid, int run, int xcd0) {
   const int b = blockIdx.x * 256 + threadIdx.x;
   if (b < grid) {
     Tile t{nullptr, nullptr, -1, 0, 0, 0, 0, 0};
-    const int xcd = b % 8, pos = b / 8;
+    const int xcd = (b + 8 - xcd0) % 8, pos = b / 8;  // counted from xcd0
     const int i = (pos / run) * (8 * run) + xcd * run + pos % run;
     if (i < n_tiles) {
       const int s0 = i * span;
@@ -153,7 +153,7 @@ extern "C" int mprgp_qp_solve_noalloc(mprgp_qp *q, const mprgp_params *params, m
   StateWords sw;
   std::memcpy(&sw, &st, sizeof(sw));
   noalloc_tables<<<(grid + 255) / 256, 256, 0, s>>>(base, d, sw, q->st, q->part, q->A->n_slices, span, n_tiles,
-                                                    grid, run);
+                                                    grid, run, ctx->tab.start.xcd());
   MPRGP_HIP(hipGetLastError());
   int steps = p.graph_steps > 0 ? p.graph_steps : 16;
   if (p.graph_steps < 0) steps = -p.graph_steps;
