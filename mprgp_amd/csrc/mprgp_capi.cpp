@@ -196,8 +196,20 @@ extern "C" int mprgp_ctx_create(int device, size_t hbm_budget_bytes, mprgp_ctx *
   c->device = device;
   c->budget = hbm_budget_bytes;
   hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_running, 2 * sizeof(int), hipHostMallocDefault);
-  if (e == hipSuccess) e = hipHostMalloc(&c->h_final, 2 * sizeof(QpState), hipHostMallocDefault);
+  // one pinned block; where the transfer part is not to be had, the host
+  // vectors are copied from where they are
+  constexpr size_t kFinal = 2 * sizeof(QpState), kRunning = 64;
+  if (e == hipSuccess) {
+    const bool whole = hipHostMalloc(&c->h_pin, kFinal + kRunning + kXferMax, hipHostMallocDefault) == hipSuccess;
+    if (!whole) {
+      (void)hipGetLastError();
+      c->h_pin = nullptr;
+      e = hipHostMalloc(&c->h_pin, kFinal + kRunning, hipHostMallocDefault);
+    }
+    c->h_final = c->h_pin;
+    c->h_running = (int *)((char *)c->h_pin + kFinal);
+    c->h_xfer = whole ? (double *)((char *)c->h_pin + kFinal + kRunning) : nullptr;
+  }
   if (e == hipSuccess) e = hipEventCreate(&c->t0);
   if (e == hipSuccess) e = hipEventCreate(&c->t1);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&c->q[0], hipEventDisableTiming);
@@ -206,11 +218,6 @@ extern "C" int mprgp_ctx_create(int device, size_t hbm_budget_bytes, mprgp_ctx *
   if (e != hipSuccess) {
     mprgp_ctx_destroy(c);
     return fail(MPRGP_EHIP, "context setup failed: %s", hipGetErrorString(e));
-  }
-  // without it the host vectors are copied from where they are
-  if (hipHostMalloc((void **)&c->h_xfer, kXferMax, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    c->h_xfer = nullptr;
   }
   int rc = c->tab.init(c);
   if (!rc) rc = noalloc_setup(device);
@@ -230,9 +237,7 @@ extern "C" void mprgp_ctx_destroy(mprgp_ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   c->tab.destroy();
   c->release(c->scratch, c->scratch_bytes);
-  if (c->h_running) (void)hipHostFree(c->h_running);
-  if (c->h_final) (void)hipHostFree(c->h_final);
-  if (c->h_xfer) (void)hipHostFree(c->h_xfer);
+  if (c->h_pin) (void)hipHostFree(c->h_pin);
   if (c->t0) (void)hipEventDestroy(c->t0);
   if (c->t1) (void)hipEventDestroy(c->t1);
   if (c->q[0]) (void)hipEventDestroy(c->q[0]);

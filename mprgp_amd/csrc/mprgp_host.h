@@ -269,8 +269,9 @@ struct mprgp_ctx {
   std::mutex amu;            // guards budget accounting (alloc/release)
   std::recursive_mutex mu;   // serialises calls that use `stream`
   mprgp::BatchTables tab;    // solve_batch's launch tables
-  int *h_running = nullptr;  // pinned, 2 slots
-  void *h_final = nullptr;   // pinned: a QP's two state copies, read back by the no-alloc solve
+  void *h_pin = nullptr;     // the context's pinned memory, holding the next two and h_xfer
+  int *h_running = nullptr;  // 2 slots
+  void *h_final = nullptr;   // a QP's two state copies, read back by the no-alloc solve
   hipEvent_t t0 = nullptr, t1 = nullptr, q[2] = {nullptr, nullptr};
   hipEvent_t ready = nullptr;  // marks the stream's work for solves on another stream
   // scratch shared by calls on this context (serialised by `mu`)
@@ -295,8 +296,9 @@ namespace mprgp {
 // copies queued on pinned memory lie between).  Calls of more than kXferMax
 // bytes copy from and to the caller's memory, where the difference is gone
 // (3.5 MB: 209 and 220 us), as they do where no pinned memory is to be had.
-// It is made with the context, whole: 0.4 ms once in a process, 12 us for a
-// context after another one.  Grown by need, a first call paid for it.
+// It is made with the context, whole, in the block of its other pinned memory
+// (a context made and closed 83 us; 134 in a block of its own, 111 to 147
+// without); grown by need, a first call paid for it.
 constexpr size_t kXferMax = (size_t)4 << 20;
 class Transfer {
  public:
