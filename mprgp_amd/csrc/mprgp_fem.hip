@@ -318,17 +318,19 @@ __global__ void __launch_bounds__(128) fem_element(int T, const int4 *__restrict
 // LDS holds are taken in runs, which keep the order of the sums.  The
 // workgroup's blocks stand by descending list length, so that the diagonal's
 // (24 tets in a Kuhn mesh, 4 to 6 elsewhere) share a wavefront.
+// HELD = false: for a body whose tet lists found no room; a contribution names
+// its tet itself, whose record is read where it lies.
 constexpr int kGroup = 256;  // blocks of A, threads
 constexpr int kHeld = 96;    // records in LDS, 264 bytes apart (40 to 112: 72-78 us; 224, two workgroups a CU: 117 us)
+template <bool HELD>
 __global__ void __launch_bounds__(kGroup) fem_blocks(long long nb, const int *__restrict__ ptr, const int *__restrict__ ctr,
                                                      const int *__restrict__ grp_ptr, const int *__restrict__ grp_tet,
                                                      const int *__restrict__ vbase, const int *__restrict__ diag_node,
                                                      const double *__restrict__ mass, double mc, double kc,
                                                      const double *__restrict__ elem, double *__restrict__ val) {
-  __shared__ double held[kHeld * (kRec + 1)];
+  __shared__ double held[HELD ? kHeld * (kRec + 1) : 1];
   const int grp = near_block(), tid = threadIdx.x;
   const long long b = (long long)grp * kGroup + tid;
-  const int t0 = grp_ptr[grp], nt = grp_ptr[grp + 1] - t0;
   int k = 0, end = 0;
   if (b < nb) {
     k = ptr[b];
@@ -337,6 +339,22 @@ __global__ void __launch_bounds__(kGroup) fem_blocks(long long nb, const int *__
   int code = k < end ? ctr[k] : INT_MAX;
   double acc[9];
   for (int e = 0; e < 9; ++e) acc[e] = 0.0;
+  auto add = [&](const double *q) {  // the contribution `code`, from its tet's record; then the next code
+    const int I = code >> 2 & 3, J = code & 3;
+    code = ++k < end ? ctr[k] : INT_MAX;
+    double uI[3], uJ[3], rr[6];
+    for (int e = 0; e < 3; ++e) {
+      uI[e] = q[3 * I + e];
+      uJ[e] = q[3 * J + e];
+    }
+    for (int e = 0; e < 6; ++e) rr[e] = q[kRecRR + e];
+    const double V = q[kRecV], lam = q[kRecV + 1], mu = q[kRecV + 2], bb = q[kRecBB + low(I, J)];
+    for (int r = 0; r < 3; ++r)
+      for (int c = 0; c < 3; ++c) acc[r * 3 + c] += stiffness(V, lam, mu, uI, uJ, rr[low(r, c)], bb, r, c) * kc;
+  };
+  if constexpr (!HELD)
+    while (k < end) add(elem + (size_t)(code >> 4) * kRec);
+  const int t0 = HELD ? grp_ptr[grp] : 0, nt = HELD ? grp_ptr[grp + 1] - t0 : 0;
   for (int base = 0; base < nt; base += kHeld) {
     const int here = min(kHeld, nt - base);
     __syncthreads();
@@ -347,20 +365,7 @@ __global__ void __launch_bounds__(kGroup) fem_blocks(long long nb, const int *__
       held[r * (kRec + 1) + e + 1] = v.y;
     }
     __syncthreads();
-    while (code >> 4 < base + here) {
-      const double *q = held + ((code >> 4) - base) * (kRec + 1);
-      const int I = code >> 2 & 3, J = code & 3;
-      code = ++k < end ? ctr[k] : INT_MAX;
-      double uI[3], uJ[3], rr[6];
-      for (int e = 0; e < 3; ++e) {
-        uI[e] = q[3 * I + e];
-        uJ[e] = q[3 * J + e];
-      }
-      for (int e = 0; e < 6; ++e) rr[e] = q[kRecRR + e];
-      const double V = q[kRecV], lam = q[kRecV + 1], mu = q[kRecV + 2], bb = q[kRecBB + low(I, J)];
-      for (int r = 0; r < 3; ++r)
-        for (int c = 0; c < 3; ++c) acc[r * 3 + c] += stiffness(V, lam, mu, uI, uJ, rr[low(r, c)], bb, r, c) * kc;
-    }
+    while (code >> 4 < base + here) add(held + ((code >> 4) - base) * (kRec + 1));
   }
   if (b >= nb) return;
   const int dn = diag_node[b];
@@ -481,7 +486,8 @@ struct mprgp_fem {
   size_t dev_bytes = 0;
   int4 *tets = nullptr;
   double *dinv = nullptr, *vol = nullptr, *lam_mu = nullptr, *node_mass = nullptr, *mass_rho = nullptr;
-  int *blk_ptr = nullptr, *blk_ctr = nullptr, *grp_ptr = nullptr, *grp_tet = nullptr, *blk_vbase = nullptr, *blk_diag = nullptr;
+  int *blk_ptr = nullptr, *blk_ctr = nullptr, *blk_vbase = nullptr, *blk_diag = nullptr;
+  int *grp_ptr = nullptr, *grp_tet = nullptr;  // null: left out (mprgp_fem_create)
   int *node_ptr = nullptr, *node_ctr = nullptr;
   double *rot = nullptr;   // per-tet rotations of the last corotational assembly
   bool rot_valid = false;
@@ -617,7 +623,10 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   for (long long b = 0; b < nb; ++b) bcnt[b + 1] += bcnt[b];
   for (int a = 0; a < N; ++a) ncnt[a + 1] += ncnt[a];
   for (int g = 0; g < runs; ++g) gptr[g + 1] += gptr[g];
-  std::vector<int> bctr(bcnt[nb]), nctr(ncnt[N]), gtet(gptr[runs]);
+  // the contributions, and behind them gptr and the tet lists, as they lie on the device
+  std::vector<int> bctr((size_t)bcnt[nb] + runs + 1 + gptr[runs]), nctr(ncnt[N]);
+  int *const gtet = bctr.data() + bcnt[nb] + runs + 1;
+  std::copy(gptr.begin(), gptr.end(), gtet - (runs + 1));
   {
     std::vector<int> bf(bcnt.begin(), bcnt.end() - 1), nf(ncnt.begin(), ncnt.end() - 1);
     std::vector<int> gf(gptr.begin(), gptr.end() - 1);
@@ -655,14 +664,24 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   f->nb = nb;
   f->density = density;
   f->min_mass = *std::min_element(mass_rho.begin(), mass_rho.end());
-  size_t bytes = 256 * 19 + sizeof(int4) * T + sizeof(double) * (9 + 1 + 2 + 9) * (size_t)T +
-                 sizeof(double) * 2 * N + sizeof(int) * ((nb + 1) + bctr.size() + 2 * nb + (N + 1) + nctr.size() + gptr.size() + gtet.size());
-  if (int rc = ctx->alloc(&f->dev, bytes)) {
-    mprgp_matrix_destroy(A);
-    delete f;
-    return rc;
+  size_t bytes = 256 * 17 + sizeof(int4) * T + sizeof(double) * (9 + 1 + 2 + 9) * (size_t)T +
+                 sizeof(double) * 2 * N + sizeof(int) * ((nb + 1) + (size_t)bcnt[nb] + 2 * nb + (N + 1) + nctr.size());
+  // the tet lists are left out where there is no room for them: the
+  // contributions then name their tets themselves
+  f->dev_bytes = bytes + sizeof(int) * (bctr.size() - bcnt[nb]);
+  const bool lists = ctx->alloc(&f->dev, f->dev_bytes) == MPRGP_OK;
+  if (!lists) {
+    f->dev_bytes = bytes;
+    if (int rc = ctx->alloc(&f->dev, bytes)) {
+      mprgp_matrix_destroy(A);
+      delete f;
+      return rc;
+    }
+    for (int g = 0; g < runs; ++g)
+      for (int k = bcnt[(size_t)g * kGroup]; k < bcnt[std::min<long long>((g + 1LL) * kGroup, nb)]; ++k)
+        bctr[k] = gtet[gptr[g] + (bctr[k] >> 4)] * 16 + (bctr[k] & 15);
+    bctr.resize(bcnt[nb]);
   }
-  f->dev_bytes = bytes;
   char *p = (char *)f->dev;
   f->tets = carve<int4>(p, T);
   f->dinv = carve<double>(p, 9 * (size_t)T);
@@ -672,8 +691,10 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   f->mass_rho = carve<double>(p, N);
   f->blk_ptr = carve<int>(p, nb + 1);
   f->blk_ctr = carve<int>(p, bctr.size());
-  f->grp_ptr = carve<int>(p, gptr.size());
-  f->grp_tet = carve<int>(p, gtet.size());
+  if (lists) {
+    f->grp_ptr = f->blk_ctr + bcnt[nb];
+    f->grp_tet = f->grp_ptr + runs + 1;
+  }
   f->blk_vbase = carve<int>(p, nb);
   f->blk_diag = carve<int>(p, nb);
   f->node_ptr = carve<int>(p, N + 1);
@@ -688,8 +709,6 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   if (!e) e = hipMemcpyAsync(f->mass_rho, mass_rho.data(), sizeof(double) * N, hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->blk_ptr, bcnt.data(), sizeof(int) * (nb + 1), hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->blk_ctr, bctr.data(), sizeof(int) * bctr.size(), hipMemcpyHostToDevice, s);
-  if (!e) e = hipMemcpyAsync(f->grp_ptr, gptr.data(), sizeof(int) * gptr.size(), hipMemcpyHostToDevice, s);
-  if (!e) e = hipMemcpyAsync(f->grp_tet, gtet.data(), sizeof(int) * gtet.size(), hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->blk_vbase, vbase.data(), sizeof(int) * nb, hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->blk_diag, diag.data(), sizeof(int) * nb, hipMemcpyHostToDevice, s);
   if (!e) e = hipMemcpyAsync(f->node_ptr, ncnt.data(), sizeof(int) * (N + 1), hipMemcpyHostToDevice, s);
@@ -752,7 +771,8 @@ int assemble_dev(mprgp_fem *f, int material, const double *xn, const double *vn,
                                               elem);
   MPRGP_HIP(hipGetLastError());
   if (!rhs_only) {
-    fem_blocks<<<(unsigned)((f->nb + kGroup - 1) / kGroup), kGroup, 0, s>>>(
+    const auto blocks = f->grp_ptr ? fem_blocks<true> : fem_blocks<false>;
+    blocks<<<(unsigned)((f->nb + kGroup - 1) / kGroup), kGroup, 0, s>>>(
         f->nb, f->blk_ptr, f->blk_ctr, f->grp_ptr, f->grp_tet, f->blk_vbase, f->blk_diag, f->mass_rho, mc, kc, elem,
         f->A->d_val);
     MPRGP_HIP(hipGetLastError());

@@ -88,3 +88,56 @@ def test_coupled_solve_without_room_for_the_one_workgroup_loop(ctx):
     with pytest.raises(M.MprgpError) as e:
         on_budget(A, b, x0, call, least - 1)
     assert e.value.code == -7
+
+
+@pytest.mark.parametrize("material", [M.LINEAR, M.COROTATIONAL])
+def test_fem_body_without_room_for_its_tet_lists(ctx, material):
+    sc = problems.beam_scene("b", 12, 4, 4, seed=3, tol=1e-8, material=material)
+    # nodes in no order, so that the lists are long
+    order = np.random.default_rng(5).permutation(sc.n_nodes)
+    X0, tets = sc.X0[order], np.argsort(order)[sc.tets].astype(np.int32)
+    x, v = 1.01 * X0.ravel(), sc.v_n[order].ravel()
+
+    filler = sp.eye(60000, format="csr")  # held while the body is made, given back before it is used
+
+    def system(room=None):
+        c = M.Context(0)
+        try:
+            c.matrix_csr(filler)
+            held = c.memory()[0]
+        finally:
+            c.close()
+        c = M.Context(0, hbm_budget=0 if room is None else held + room)
+        try:
+            fill = c.matrix_csr(filler)
+            before = c.memory()[0]
+            fem = M.Fem(c, X0, tets, sc.young, sc.poisson, sc.density)
+            made = c.memory()[0]
+            fill.close()
+            q = fem.matrix.qp()
+            fem.set_damping(0.1, 0.02)
+            fem.assemble(q, x, v, sc.gravity, sc.h, material)
+            rowptr, colidx, blocks = fem.matrix.get_bsr3()
+            return made - before, (rowptr, colidx, blocks, q.get_rhs())
+        finally:
+            c.close()
+    made, want = system()
+    c = M.Context(0)
+    try:
+        empty = c.memory()[0]
+        P = sp.bsr_matrix((np.ones((len(want[1]), 3, 3)), want[1], want[0]))
+        A = c.matrix_csr((P + sp.eye(P.shape[0])).tocsr())
+        matrix = c.memory()[0] - empty
+        A.close()
+    finally:
+        c.close()
+    N, T, nb = sc.n_nodes, len(tets), len(want[1])
+    body = 256 * 17 + 16 * T + 8 * 21 * T + 16 * N + 4 * (nb + 1 + 16 * T + 2 * nb + N + 1 + 4 * T)
+    assert made > matrix + body  # the lists
+    least, got = system(matrix + body)
+    assert least == matrix + body
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(a, b)
+    with pytest.raises(M.MprgpError) as e:
+        system(matrix + body - 1)
+    assert e.value.code == -7
