@@ -43,12 +43,12 @@ SPW_CANDIDATES = [1, 2]
 # tiles, one workgroup per CU).
 TAIL_CANDIDATES = [0, 64, 128, 512, 1024, 2048]
 
-# Placements of the tiles on the 8 XCDs tried last (0: runs of 4 tiles
+# Placements of the tiles on the 8 XCDs tried last (0: runs of 4 to 32 tiles
 # rotating over the XCDs, 1: one contiguous chunk of each QP per XCD).
 LAYOUT_CANDIDATES = [0, 1]
 
 # Bumped whenever the step kernel changes in a way that moves the best shape.
-CACHE_VERSION = 8
+CACHE_VERSION = 9
 
 
 def cache_path():
