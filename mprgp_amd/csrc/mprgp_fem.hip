@@ -187,17 +187,17 @@ __device__ void polar_rotation(const double *F, double *R) {
 // rot: per-tet rotations, [entry][tet].  corot && !lag: R is the polar
 // rotation of F and is stored; corot && lag: R is the stored rotation of the
 // last full assembly (the element is then linear in x with exactly the
-// stiffness of that assembly).  rhs_only skips the stiffness blocks.
-// Outputs (FEMSystem::buildSystem, FEMSystem.cpp:167-192): the stiffness
-// blocks times kc = h^2 + h alpha_m, the force times h^2, and with damp set
-// the unscaled K_e c_e for c = (x_n - x1) h (the stiffness-damping term, CRHS).
+// stiffness of that assembly).  rhs_only skips the stiffness records.
+// Outputs (FEMSystem::buildSystem, FEMSystem.cpp:167-192): the record of K_e,
+// the force times h^2, and with damp set the unscaled K_e c_e for
+// c = (x_n - x1) h (the stiffness-damping term, CRHS).
 __global__ void __launch_bounds__(128) fem_element(int T, const int4 *__restrict__ tets,
                                                    const double *__restrict__ dinv,
                                                    const double *__restrict__ vol,
                                                    const double *__restrict__ lam_mu,
                                                    const double *__restrict__ x,
                                                    const double *__restrict__ xn, int corot, int lag,
-                                                   int rhs_only, int damp, double kc, double h2, double h,
+                                                   int rhs_only, int damp, double h2, double h,
                                                    double *__restrict__ rot, double *__restrict__ out) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= T) return;
@@ -323,9 +323,10 @@ __global__ void __launch_bounds__(128) fem_element(int T, const int4 *__restrict
 constexpr int kGroup = 256;  // blocks of A, threads
 constexpr int kHeld = 96;    // records in LDS, 264 bytes apart (40 to 112: 72-78 us; 224, two workgroups a CU: 117 us)
 template <bool HELD>
-__global__ void __launch_bounds__(kGroup) fem_blocks(long long nb, const int *__restrict__ ptr, const int *__restrict__ ctr,
-                                                     const int *__restrict__ grp_ptr, const int *__restrict__ grp_tet,
-                                                     const int *__restrict__ vbase, const int *__restrict__ diag_node,
+__global__ void __launch_bounds__(kGroup) fem_blocks(long long nb, const int *__restrict__ ptr,
+                                                     const int *__restrict__ ctr, const int *__restrict__ grp_ptr,
+                                                     const int *__restrict__ grp_tet, const int *__restrict__ vbase,
+                                                     const int *__restrict__ diag_node,
                                                      const double *__restrict__ mass, double mc, double kc,
                                                      const double *__restrict__ elem, double *__restrict__ val) {
   __shared__ double held[HELD ? kHeld * (kRec + 1) : 1];
@@ -587,7 +588,8 @@ extern "C" int mprgp_fem_create(mprgp_ctx *ctx, int N, int T, const int *tets_in
   // and more count as equal), and each run's tets, ascending, by whose place
   // in that list (the run's last tet so far) a contribution names its tet.
   // Filled tet by tet, so nothing is sorted: sorting the blocks and the tets
-  // of each run made a body of 44,541 nodes 74 ms instead of 64, one of 15,975 20.4 instead of 17.3.
+  // of each run made a body of 44,541 nodes 74 ms instead of 64, one of 15,975
+  // 20.4 instead of 17.3.
   auto blk_of = [&](int a, int b) {
     auto it = std::lower_bound(colidx.begin() + rowptr[a], colidx.begin() + rowptr[a + 1], b);
     return (int)(it - colidx.begin());
@@ -767,8 +769,7 @@ int assemble_dev(mprgp_fem *f, int material, const double *xn, const double *vn,
   const int damp = f->alpha_m != 0.0 ? 1 : 0;
   const int corot = material == MPRGP_COROTATIONAL;
   fem_element<<<(T + 127) / 128, 128, 0, s>>>(T, f->tets, f->dinv, f->vol, f->lam_mu, x1, xn, corot,
-                                              rhs_only ? 1 : 0, rhs_only ? 1 : 0, damp, kc, h2, bdt, f->rot,
-                                              elem);
+                                              rhs_only ? 1 : 0, rhs_only ? 1 : 0, damp, h2, bdt, f->rot, elem);
   MPRGP_HIP(hipGetLastError());
   if (!rhs_only) {
     const auto blocks = f->grp_ptr ? fem_blocks<true> : fem_blocks<false>;

@@ -318,7 +318,8 @@ struct General {
   int loop_on_device(double alpha_bar, double tol, int max_it, bool pre, GenState *st) {
     const mprgp_matrix *A = q->A;
     const GenArgs a{n, m, A->n_nodes, A->n_slices, A->d_sl_off, A->d_col, A->d_val, dinv, b, x, g, p, z, phi, beta,
-                    y, gp, t, t2, t3, tl, jp, jc, tp, tc, jv, tv, d_c, d_ctl->face, jslot(0), jslot(1), lam, lam + m + 1, part,
+                    y, gp, t, t2, t3, tl, jp, jc, tp, tc, jv, tv, d_c, d_ctl->face, jslot(0), jslot(1), lam,
+                    lam + m + 1, part,
                     (int)big_row.size() / kGenBlock, (int)one_row.size(), d_big_row, d_one_row, d_big_g, d_one_g,
                     alpha_bar, tol, max_it, pre, kGenChunk, &d_ctl->st};
     h_ctl->args = a;

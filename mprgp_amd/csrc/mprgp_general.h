@@ -7,12 +7,14 @@ namespace mprgp {
 
 // Rows of the largest component (rows that share nodes) the one-workgroup loop
 // takes: a vertex-triangle contact row and the plane rows of its four nodes
-// are five.  A component's QP runs in one thread's registers.
+// are five.  A component's QP runs in one wavefront's registers, its block of
+// J J^T one entry a lane.
 constexpr int kGenBlock = 6;
 // Nodes of the largest system: the vector a product gathers from is 24 bytes
-// a node of the 64 KB a kernel declares.  There the loop is still the faster
-// one, 271 ms against 570 ms from the host over 1,001 iterations at 2,499
-// nodes, but its products with A, on one CU, grow with the matrix.
+// a node of the 64 KB a kernel declares.  There the loop can still be the
+// faster one (a beam of 2,499 nodes, 2,511 rows, 271 ms against 570 ms from
+// the host over 1,001 iterations), but its products with A, on one CU, grow
+// with the matrix.
 constexpr int kGenMaxNodes = 2600;
 constexpr int kGenMaxRows = 16384;  // some two rows per entry of the largest vector
 // What the one-workgroup loop gains on the host-driven one, microseconds an
@@ -21,11 +23,11 @@ constexpr int kGenMaxRows = 16384;  // some two rows per entry of the largest ve
 // takes for the vectors, the matrix (its load path) and the components of
 // several rows (a wavefront each, 16 at a time; the host factors a block in
 // less than a wavefront does).  The loop is taken where the estimate is
-// positive.  Fitted low to 360 pairs of both loops' times (100 to 2,600 nodes, 3 to
-// 300 blocks a row, 0 to 512 components of 1 to 6 rows, none to all of their
-// rows active, CG and expansion steps), so that none of those estimated
-// positive was slower than from the host: 2,600 nodes, host / one workgroup:
-// 3 blocks a row, 8 pairs of rows 202 / 95 us, 256 pairs 313 / 339, 512
+// positive.  Fitted low to 360 pairs of both loops' times (100 to 2,600 nodes,
+// 3 to 300 blocks a row, 0 to 512 components of 1 to 6 rows, none to all of
+// their rows active, CG and expansion steps), so that none of those estimated
+// positive was slower than from the host.  2,600 nodes, host / one workgroup,
+// 3 blocks a row: 16 pairs of rows 202 / 107 us, 256 pairs 313 / 339, 512
 // components of six 800 / 1,473; 27 blocks a row, 8 pairs 210 / 242.  A beam
 // of 525 nodes with 525 ground rows and 12 contacts 344 / 105.
 constexpr double kGenGain = 145.0, kGenRowGain = 0.07, kGenNodeCost = 0.03, kGenSlotCost = 0.0019;

@@ -1,7 +1,8 @@
 // mprgp_general_dev.hip -- the main loop of the coupled-row solve
 // (MPRGPMonotonic::solve with GeneralConProjector, MPRGPSolver.h:412-454,
 // MPRGPProjection.h:400-520) in one workgroup, for systems of at most
-// kGenMaxNodes nodes whose rows form components of at most kGenBlock rows.
+// kGenMaxNodes nodes whose rows form components of at most kGenBlock rows,
+// where one CU is the faster way (mprgp_general.h).
 //
 // Driven from the host, an iteration is about 50 launches of small kernels and
 // five waits, nearly all of its time.  Here the vectors stay where they are
@@ -48,7 +49,8 @@ using Shared = __attribute__((address_space(3))) Block;
 template <class T>
 __device__ __forceinline__ T *uniform(T *p) {  // p, the same in all lanes, in scalar registers
   const auto u = (unsigned long long)p;
-  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u), hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
   return (T *)((unsigned long long)hi << 32 | lo);
 }
 template <class T>
@@ -545,7 +547,8 @@ __global__ void __launch_bounds__(kThreads) general_loop(const GenArgs *args) {
   Args *a = (Args *)args;
   const int tid = threadIdx.x, n = a->n, max_it = a->max_it;
   const double ab = a->alpha_bar, tol = a->tol;
-  double *x_ = a->x, *y_ = a->y, *g_ = a->g, *p_ = a->p, *z_ = a->z, *beta_ = a->beta, *ap_ = a->ap, *t_ = a->t, *t2_ = a->t2;
+  double *x_ = a->x, *y_ = a->y, *g_ = a->g, *p_ = a->p, *z_ = a->z, *beta_ = a->beta;
+  double *ap_ = a->ap, *t_ = a->t, *t2_ = a->t2;
   const auto x = mem(x_), y = mem(y_), g = mem(g_), p = mem(p_), z = mem(z_), phi = mem(a->phi);
   const auto beta = mem(beta_), ap = mem(ap_), t = mem(t_), t2 = mem(t2_);
   const bool pre = a->pre;

@@ -18,9 +18,8 @@
 // highest level among the nodes it couples to that come before it), and one
 // workgroup runs the levels in order with a barrier between them, x in an
 // LDS ring where the levels' reach allows (ica_sweep_ring).  Every node then
-// sees exactly the new and old values the sequential sweep gives
-// it, so the sweep is the reference's, not a multicolour variant with other
-// iterates.  Each row adds its terms in the order of its blocks (the input's
+// sees exactly the new and old values the sequential sweep gives it, so the
+// sweep is the reference's, not a multicolour variant with other iterates.  Each row adds its terms in the order of its blocks (the input's
 // column order), singly rounded, as the oracle does.
 #include <hip/hip_runtime.h>
 

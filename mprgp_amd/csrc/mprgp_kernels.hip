@@ -304,8 +304,9 @@ constexpr bool split_trial(int ts, int spw, int ub) { return ub == kUnrollTail &
 // launch writes; NV = 2 also gives A x.  A round first loads its columns' x,
 // p and row flags, then, on the lanes that have a flagged column, all of the
 // round's row data at once (loading every column's row data with the first
-// loads measured the same, also where every node has a row).  Forming P(w) here replaces an elementwise launch
-// before the product.
+// loads measured the same, also where every node has a row).  Forming P(w)
+// here replaces an elementwise launch before the product (split_trial: not
+// everywhere).
 template <int NV, int U, bool NT, bool STEP, class C, class T>
 __device__ __forceinline__ void spmv_proj(const QpDev &q, const Vecs<T> &v, const C *col, const double *x,
                                           double alpha, int s, int lane, V3 (&acc)[NV]) {
@@ -1060,7 +1061,8 @@ __device__ __forceinline__ void row_work(const QpDev &q, const Vecs<T> &vin, int
       if constexpr (!std::is_same_v<T, double>) break;
       V3 acc[1];
       if constexpr (SPLIT)
-        spmv_row<1, UB, NT>(q.sl_off, cols<C16>(q), v.val, s, lane, [&](int j, V3 (&xs)[1]) { xs[0] = ld3(v.py, j); }, acc);
+        spmv_row<1, UB, NT>(q.sl_off, cols<C16>(q), v.val, s, lane, [&](int j, V3 (&xs)[1]) { xs[0] = ld3(v.py, j); },
+                            acc);
       else
         spmv_proj<1, proj_unroll(UB), NT, true>(q, v, cols<C16>(q), xc, st.alpha, s, lane, acc);
       const V3 xr = ld3(xc, r), pr = ld3(v.p, r);
@@ -1427,7 +1429,7 @@ __global__ void __launch_bounds__(TS * kSlice, UB == kUnroll ? MPRGP_STEP_MIN_WA
     mprgp_step(const QpDev *__restrict__ qps,
                                                            const Tile *__restrict__ tiles,
                                                            int *running, int parity) {
-  __shared__ double red[TS > 1 ? TS : 1][kNumPart];
+  __shared__ double red[TS][kNumPart];
   __shared__ QpState sst;
   const int wave = threadIdx.x / kSlice;
   const int lane = threadIdx.x % kSlice;
