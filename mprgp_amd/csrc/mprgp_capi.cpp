@@ -1244,7 +1244,7 @@ extern "C" int mprgp_qp_get_rows(mprgp_qp *q, int cap, int *m, int *node, double
 namespace mprgp {
 
 namespace {
-// live drivers per XCD of each device; never freed, a context may outlive it
+// XcdStarts taken per XCD of each device; never freed, a context may outlive it
 std::mutex &start_mu() {
   static std::mutex *m = new std::mutex();
   return *m;

@@ -126,10 +126,10 @@ int build_matrix(mprgp_ctx *ctx, int n_nodes, const int *rowptr, const int *coli
 
 constexpr int kXcds = 8, kXcdCus = 32;
 
-// The XCD that the first tiles of a driver's launches stand on: of the
-// device's, one that the fewest live drivers have, halves apart first.  A
-// launch of few tiles stands on few XCDs (xcd_run), and drivers whose solves
-// run at the same time would share those while others idle.  Two contexts
+// The XCD that the first tiles of a context's or an engine's launches stand
+// on: of the device's, one that the fewest of those alive have, halves apart
+// first.  A launch of few tiles stands on few XCDs (xcd_run), and contexts
+// that solve at the same time would share those while others idle.  Two contexts
 // solving 7,139 nodes (112 tiles, four XCDs) with the power method: 12.1 ms a
 // solve on the same four, 10.0 apart, 11.1 in runs of 4 over all eight; 4,100
 // nodes 10.3, 8.6 and 10.4; three contexts, which have to overlap, 12.8, 12.4

@@ -1,4 +1,4 @@
-// Where the launches of concurrent drivers start (XcdStart): the first eight
+// Where the launches of concurrent contexts start (XcdStart): the first eight
 // on XCDs of their own, halves apart first, the next on the first free again,
 // and each device counted by itself.
 #include <cstdio>
@@ -22,7 +22,7 @@ int main() {
     s.back()->take(0);
     seen |= 1u << s.back()->xcd();
   }
-  expect(seen == 0xff, "eight drivers, eight XCDs");
+  expect(seen == 0xff, "eight contexts, eight XCDs");
   expect(s[0]->xcd() == 0 && s[1]->xcd() == 4, "the second half the card away");
   expect((s[2]->xcd() & 1) == 0 && (s[3]->xcd() & 1) == 0, "then quarters");
   XcdStart other;
@@ -41,7 +41,7 @@ int main() {
   for (int i = 0; i < 1000; ++i) {
     XcdStart t;
     t.take(1);
-    expect(t.xcd() == 4, "short-lived drivers leave nothing");
+    expect(t.xcd() == 4, "short-lived contexts leave nothing");
   }
   return fails != 0;
 }

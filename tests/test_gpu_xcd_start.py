@@ -1,4 +1,4 @@
-"""The XCD a driver's launches start on changes no result: solves on nine
+"""The XCD a context's launches start on changes no result: solves on nine
 contexts alive at once (one more than the XCDs), one after the other and all
 at the same time, from the context's tables and from those built on the
 device, and through an engine beside them."""
